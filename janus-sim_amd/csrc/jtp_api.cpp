@@ -111,8 +111,106 @@ static double split_excess_x3(double x) {
     return (split_direct(x, true) - 1.0) / (x * x * x);
 }
 
+// The same factors in extended precision for the FP64 walk's fits.  split_excess: (S - 1) / x^3 (erfc +
+// Gaussian) or (S - 1) / x (erfc only), by its series below x = 1/2, where the direct form cancels.
+static long double split_direct_l(long double x, bool gauss) {
+    return erfcl(x) + (gauss ? 2.0L * x / sqrtl((long double)M_PIl) * expl(-x * x) : 0.0L);
+}
+static long double split_excess_l(long double x, bool gauss) {
+    if (x >= 0.5L) return (split_direct_l(x, gauss) - 1.0L) / (gauss ? x * x * x : x);
+    // erf(x) = 2/sqrt(pi) sum (-1)^n x^{2n+1} / (n! (2n+1)); with the Gaussian term, see split_excess_x3
+    const long double x2 = x * x;
+    long double term = 1.0L, sum = 0.0L;  // gauss: x^{2n-2} / n! from n = 1; erfc only: x^{2n} / n! from n = 0
+    for (int n = gauss ? 1 : 0; n < 40; ++n) {
+        if (n > (gauss ? 1 : 0)) term *= x2 / n;
+        const long double w = gauss ? 2.0L * n / (2.0L * n + 1.0L) : -1.0L / (2.0L * n + 1.0L);
+        sum += (n & 1) ? -term * w : term * w;
+    }
+    return 2.0L / sqrtl((long double)M_PIl) * sum;
+}
+
+// Degree-deg Chebyshev interpolant of f on [a, b] as monomial coefficients of t = 2 (v - a) / (b - a) - 1, in
+// extended precision, rounded once.
+template <typename F>
+static void cheb_fit_l(long double a, long double b, int deg, double* out, F f) {
+    const int N = deg + 1;
+    std::vector<long double> fv(N), mono(N, 0.0L), t0(N, 0.0L), t1(N, 0.0L), t2(N, 0.0L);
+    for (int k = 0; k < N; ++k) fv[k] = f(a + 0.5L * (b - a) * (cosl((long double)M_PIl * (k + 0.5L) / N) + 1.0L));
+    t0[0] = 1.0L;
+    if (N > 1) t1[1] = 1.0L;
+    for (int j = 0; j < N; ++j) {
+        long double s = 0;
+        for (int k = 0; k < N; ++k) s += fv[k] * cosl((long double)M_PIl * j * (k + 0.5L) / N);
+        s *= (j == 0 ? 1.0L : 2.0L) / N;
+        for (int d = 0; d < N; ++d) mono[d] += s * t0[d];
+        for (int d = 0; d < N; ++d) t2[d] = -t0[d] + (d > 0 ? 2.0L * t1[d - 1] : 0.0L);  // T_{j+2}
+        t0.swap(t1);
+        t1.swap(t2);
+    }
+    for (int d = 0; d < N; ++d) out[d] = (double)mono[d];
+}
+
+// The FP64 fits in units of 2 r_s (x^2 for v): they depend on the law alone, so they are made once per process (0.4
+// ms) and scaled per context.  cut[i] covers sources cut at x <= kFit64Cut[i]; ok[i]: it and the other two are
+// within kFit64Tol of the law, relative to the Newtonian pair force.
+constexpr int kFit64Cuts = 2;
+constexpr double kFit64Cut[kFit64Cuts] = {2.3, 2.7};
+struct UnitFit64 {
+    double cut[kFit64Cuts][kFit64Pair + 1], tail[kFit64Tail + 1], far[kFit64Far + 1];
+    bool ok[kFit64Cuts];
+    explicit UnitFit64(bool gauss) {
+        auto excess = [&](long double y) { return split_excess_l(sqrtl(y), gauss); };
+        auto whole = [&](long double y) { return split_direct_l(sqrtl(y), gauss) / (y * sqrtl(y)); };
+        const long double y1 = (long double)kFit64X1 * kFit64X1, y2 = (long double)kFit64X2 * kFit64X2;
+        auto err = [&](long double a, long double b, int deg, const double* cf, bool full) {
+            long double worst = 0;
+            for (int i = 0; i <= 200; ++i) {
+                const long double y = a + (b - a) * (i + 0.01L) / 200.02L, t = 2.0L * (y - a) / (b - a) - 1.0L;
+                long double p = cf[deg];
+                for (int d = deg - 1; d >= 0; --d) p = p * t + cf[d];
+                const long double w = full || gauss ? y * sqrtl(y) : sqrtl(y);  // to the Newtonian force
+                worst = std::max(worst, fabsl(p - (full ? whole(y) : excess(y))) * w);
+            }
+            return worst;
+        };
+        cheb_fit_l(0.0L, y1, kFit64Tail, tail, excess);
+        cheb_fit_l(y1, y2, kFit64Far, far, whole);
+        const bool rest = err(0.0L, y1, kFit64Tail, tail, false) < kFit64Tol && err(y1, y2, kFit64Far, far, true) < kFit64Tol;
+        for (int i = 0; i < kFit64Cuts; ++i) {
+            const long double yp = (long double)kFit64Cut[i] * kFit64Cut[i];
+            cheb_fit_l(0.0L, yp, kFit64Pair, cut[i], excess);
+            ok[i] = rest && err(0.0L, yp, kFit64Pair, cut[i], false) < kFit64Tol;
+        }
+    }
+};
+
+static void make_split_poly64(Ctx& c) {
+    SplitPoly64& q = c.poly64;
+    q = SplitPoly64{};
+    const bool gauss = c.p.split_mode == JTP_SPLIT_ERFC_GAUSS;
+    static const UnitFit64 unit_gauss(true), unit_erfc(false);
+    const UnitFit64& u = gauss ? unit_gauss : unit_erfc;
+    const double ci = 0.5 / c.p.r_s, ci3 = ci * ci * ci;
+    const double xp = std::sqrt(c.p.r_cut * c.p.r_cut + c.p.softening * c.p.softening) * ci * (1.0 + 1e-12);
+    int k = 0;
+    while (k < kFit64Cuts && !(xp <= kFit64Cut[k])) ++k;
+    if (k == kFit64Cuts || !u.ok[k]) return;
+    for (int d = 0; d <= kFit64Pair; ++d) q.cp[d] = u.cut[k][d] * (gauss ? ci3 : ci);
+    for (int d = 0; d <= kFit64Tail; ++d) q.ct[d] = u.tail[d] * (gauss ? ci3 : ci);
+    for (int d = 0; d <= kFit64Far; ++d) q.cg[d] = u.far[d] * ci3;
+    const double c2 = ci * ci, y1 = kFit64X1 * kFit64X1, y2 = kFit64X2 * kFit64X2;
+    q.sp = 2.0 * c2 / (kFit64Cut[k] * kFit64Cut[k]);
+    q.st = 2.0 * c2 / y1;
+    q.sg = 2.0 * c2 / (y2 - y1);
+    q.og = 2.0 * y1 / (y2 - y1) + 1.0;
+    q.v1 = y1 / c2;
+    q.v2 = y2 / c2;
+    q.ok = std::isfinite(ci3) && ci3 > 1e-280 && std::isfinite(q.v2) ? 1 : 0;
+}
+
 void make_split_poly(Ctx& c) {
     if (!(c.p.r_s > 0)) return;
+    if (c.p.precision == JTP_FP64 && c.p.split_mode != JTP_SPLIT_POLY4) make_split_poly64(c);
     const double rho_max = std::sqrt(c.p.r_cut * c.p.r_cut + c.p.softening * c.p.softening);
     const double Xp = rho_max / (2.0 * c.p.r_s) * 1.0001 + 1e-12;
     const double Xm = Xp * (1.0 + std::sqrt(3.0) * c.p.theta);
@@ -359,6 +457,11 @@ int jtp_create(const jtp_params* p, jtp_ctx** out) {
     if (e == hipSuccess) e = dalloc(c.dev_step, 1);
     if (e == hipSuccess) e = dalloc(c.diag_scratch, kDiagScratch);
     if (e == hipSuccess) e = hipHostMalloc((void**)&c.host_step, sizeof(StepParams), 0);
+    make_split_poly(c);
+    if (p->precision == JTP_FP64) {  // the walk's polynomials
+        if (e == hipSuccess) e = dalloc(c.dev_fit64, 1);
+        if (e == hipSuccess) e = hipMemcpy(c.dev_fit64, &c.poly64, sizeof(SplitPoly64), hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess) e = pm_tables(c);
     if (e == hipSuccess) {
         for (int i = 0; i < 10 && e == hipSuccess; ++i) e = hipEventCreate(&c.ev[i]);
@@ -374,7 +477,6 @@ int jtp_create(const jtp_params* p, jtp_ctx** out) {
         jtp_destroy(h);
         return JTP_ERR_ALLOC;
     }
-    make_split_poly(c);
     *out = h;
     return JTP_OK;
 }
@@ -389,7 +491,7 @@ int jtp_destroy(jtp_ctx* h) {
     void* ptrs[] = {c.rho, c.phi, c.rho2, c.phi2, c.grad, c.grad2, c.spec, c.twiddle, c.gtab, c.cell_start,
                     c.tile_start, c.dep_tbuf,
                     c.cell4, c.cellnode, c.dev_counters, c.dev_inter, c.dense_slot, c.dev_step, c.diag_scratch,
-                    c.pot_short, c.acc_scratch, c.kself, c.seg};
+                    c.pot_short, c.acc_scratch, c.kself, c.seg, c.dev_fit64};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c.host_pinned) (void)hipHostFree(c.host_pinned);

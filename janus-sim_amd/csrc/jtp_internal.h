@@ -92,6 +92,27 @@ struct SplitPoly {
     float cm[kPolyDeg + 1];
 };
 
+// Polynomials of the FP64 walk's erfc laws, v = rho^2 = r^2 + eps^2, x = rho / (2 r_s).  S - 1 is x^3 (erfc +
+// Gaussian) or x (erfc only) times an entire function of x^2, so S / rho^3 = 1 / rho^3 + H(v) or
+// 1 / rho^3 + E(v) / rho^2 with H, E polynomials to double precision:
+//  * cp: sources cut at r_cut (x <= 2.3, or 2.7 for r_cut above 4.6 r_s);
+//  * ct on [0, v1], x(v1) = kFit64X1 (1.8 r_cut at the default r_cut = 4.5 r_s): monopoles of nodes that straddle r_cut;
+//  * cg: S / rho^3 itself on [v1, v2], x(v2) = kFit64X2, where S < 1e-16; zero beyond.
+// `ok`: every fit is within kFit64Tol of the law, relative to the Newtonian pair force (r_cut up to 5.4 r_s);
+// otherwise the walk calls erfc and exp.
+constexpr int kFit64Pair = 20, kFit64Tail = 30, kFit64Far = 25;
+constexpr double kFit64X1 = 4.0, kFit64X2 = 6.2;
+constexpr double kFit64Tol = 1e-15;
+struct SplitPoly64 {
+    double cp[kFit64Pair + 1];
+    double ct[kFit64Tail + 1];
+    double cg[kFit64Far + 1];
+    double sp, st;        // t = v * s - 1 of cp and ct
+    double sg, og;        // t = v * sg - og of cg
+    double v1, v2;
+    int32_t ok;
+};
+
 // Lanes of a wavefront that share one walk target: groups of <= 16 targets use 4 lanes per
 // target, <= 32 use 2, larger groups 1.
 inline int lanes_per_target(int group_size) { return group_size <= 16 ? 4 : (group_size <= 32 ? 2 : 1); }
@@ -169,6 +190,8 @@ struct Ctx {
     void *gtab = nullptr;            // real 2G: per-axis window/Gaussian factor, k_i^2
     void *pm_acc = nullptr;          // real 3n (sorted order)
     SplitPoly poly{};
+    SplitPoly64 poly64{};
+    SplitPoly64* dev_fit64 = nullptr;  // FP64 contexts: device copy of poly64
     float poly_tscale = 0.0f;    // particles: t = rho^2 * poly_tscale - 1 (erfc + Gaussian), rho * poly_tscale - 1
     float poly_tscale_m = 0.0f;  // monopoles
     float poly_rho2_tail = 0.0f; // erfc + Gaussian monopoles: rho^2 beyond which the force is dropped
