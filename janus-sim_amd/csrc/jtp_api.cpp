@@ -1230,7 +1230,7 @@ int jtp_ensemble_create(int32_t n_boxes, const jtp_params* params, const double*
     const size_t ab = walk_args_bytes() * (size_t)n_boxes;
     if (er == hipSuccess) er = hipHostMalloc((void**)&e->h_args, ab, hipHostMallocDefault);
     if (er == hipSuccess) er = hipMalloc(&e->d_args, ab);
-    if (er == hipSuccess) er = hipMalloc((void**)&e->d_ctrl, sizeof(int32_t) * (size_t)n_boxes * (2 + kXcds));
+    if (er == hipSuccess) er = hipMalloc((void**)&e->d_ctrl, sizeof(int32_t) * (size_t)n_boxes * (size_t)walk_ctrl_size(1));
     if (er != hipSuccess) {
         (void)hipGetLastError();
         jtp_ensemble_destroy(e);
@@ -1300,7 +1300,7 @@ static int ens_enqueue(jtp_ensemble* e, const int64_t* n, const uint32_t* const*
         const int m = launches[i].second;
         ENS_HIP(e, walk_boxes((const unsigned char*)e->d_args + ab * launches[i].first, m, e->d_ctrl + ctrl,
                               items[i], keys[i], s));
-        ctrl += (size_t)m + 1 + kXcds;
+        ctrl += (size_t)walk_ctrl_size(m);
     }
     for (int b : batched) {
         int rc = enqueue_status(e->boxes[b]->c, n[b], s);

@@ -35,8 +35,9 @@ constexpr int kXcds = 8;             // MI355X accelerator complex dies; workgro
 constexpr int kCtrNGroups = 0, kCtrErr = 1, kCtrDense = 3, kCtrInterp = 4;  // kCtrInterp: 3 words
 constexpr int kCtrRounds = 8;                       // [0] global frontier size, [kMaxRounds+1] root flag
 constexpr int kCtrRoot = kCtrRounds + kMaxRounds + 1;
-constexpr int kCtrXcd = kCtrRounds + kMaxRounds + 4;  // kXcds walk-queue heads
-constexpr int kCtrTotal = kCtrXcd + kXcds + 4;
+constexpr int kCtrXcd = 192;                        // kXcds walk-queue heads, kCtrXcdStride apart
+constexpr int kCtrXcdStride = 64;                   // 256 bytes: their atomics do not share a line
+constexpr int kCtrTotal = kCtrXcd + kXcds * kCtrXcdStride;
 
 // ---------------------------------------------------------------- small types
 template <typename R> struct Cplx { R x, y; };
@@ -273,7 +274,10 @@ hipError_t pm_tables(Ctx& c);                                      // twiddles +
 hipError_t walk(Ctx& c, int64_t n, void* acc_out, hipStream_t s, double* pot = nullptr);
 // One walk launch over several boxes: each box's arguments (walk_args_bytes() each, filled on the
 // host by walk_fill_args after its build is enqueued) in device memory; boxes with equal
-// walk_batch_key share a launch.  d_ctrl holds nbox + 1 + kXcds int32 (group offsets, queue heads).
+// walk_batch_key share a launch.  d_ctrl holds walk_ctrl_size(nbox) int32: the group offsets, padded to
+// a head's stride (walk_heads), then the queue heads.
+inline int64_t walk_heads(int64_t nbox) { return (nbox + kCtrXcdStride) / kCtrXcdStride * kCtrXcdStride; }
+inline int64_t walk_ctrl_size(int64_t nbox) { return walk_heads(nbox) + kXcds * kCtrXcdStride; }
 size_t walk_args_bytes();
 void walk_fill_args(Ctx& c, int64_t n, void* acc_out, void* dst);
 int walk_batch_key(const Ctx& c);

@@ -483,7 +483,7 @@ __global__ __launch_bounds__(256) void k_group_offsets(const int32_t* __restrict
         counters[kCtrNGroups] = (int32_t)tot;
         counters[kCtrErr] = 0;
     }
-    if (tid < kXcds) counters[kCtrXcd + tid] = 0;  // walk queue heads
+    if (tid < kXcds) counters[kCtrXcd + tid * kCtrXcdStride] = 0;  // walk queue heads
 }
 
 __global__ void k_groups(const int32_t* __restrict__ cell4, const int32_t* __restrict__ goff, int gs,
