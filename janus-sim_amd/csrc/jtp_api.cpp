@@ -238,8 +238,7 @@ void make_split_poly(Ctx& c) {
 
 static void free_particle_buffers(Ctx& c) {
     void* ptrs[] = {c.keys0, c.keys1, c.vals0, c.vals1, c.hist, c.hist_blk, c.parts, c.node_geo, c.node_kids,
-                    c.up, c.flags, c.node_sum, c.node_mono, c.groups, c.pm_acc,
-                    c.frontier0, c.frontier1, c.dense_list, c.dense_corner, c.interp_list, c.dep_chunks,
+                    c.node_sum, c.node_mono, c.groups, c.pm_acc, c.bt_count, c.dense_list, c.dense_corner, c.interp_list, c.dep_chunks,
                     c.dep_cbuf};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -249,9 +248,8 @@ static void free_particle_buffers(Ctx& c) {
     c.parts = nullptr;
     c.node_geo = nullptr;
     c.node_kids = nullptr;
-    c.up = nullptr;
-    c.flags = nullptr;
-    c.frontier0 = c.frontier1 = c.dense_list = nullptr;
+    c.bt_count = nullptr;
+    c.dense_list = nullptr;
     c.dense_corner = nullptr;
     c.interp_list = nullptr;
     c.dep_chunks = nullptr;
@@ -282,10 +280,7 @@ static int ensure_capacity(Ctx& c, int64_t n) {
     chk(dalloc(c.parts, cap));
     chk(dalloc(c.node_geo, 2 * cap));
     chk(dalloc(c.node_kids, cap));
-    chk(dalloc(c.up, cap));
-    chk(dalloc(c.flags, cap));
-    chk(dalloc(c.frontier0, cap));
-    chk(dalloc(c.frontier1, cap));
+    chk(dalloc(c.bt_count, (size_t)bt_count_size(cap)));
     chk(dalloc(c.interp_list, (size_t)interp_list_size(c.G3(), cap)));
     if (c.p.precision == JTP_FP64) {  // dense-cell pre-reduction of the gather deposit
         chk(dalloc(c.dense_list, cap / kDenseCell + 1));
@@ -526,7 +521,7 @@ int jtp_set_species_mass(jtp_ctx* h, double m_plus, double m_minus_abs) {
 static int enqueue_prep(Ctx& c, int64_t n, const uint32_t* d_pos, const int8_t* d_species, hipStream_t s,
                         bool timed) {
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[0], s));
-    JTP_HIP(&c, launch_fill_i32((int32_t*)c.dev_inter, 4, 0, s));
+    JTP_HIP(&c, launch_reset(c, s));
     // the packed records live in the node-sum buffer, which the tree build (after the gather) overwrites
     uint4* rec = (uint4*)c.node_sum;
     JTP_HIP(&c, launch_morton_keys(d_pos, d_species, c.keys0, c.vals0, rec, n, s));
@@ -1052,6 +1047,7 @@ int jtp_stage_copy(jtp_ctx* h, int32_t stage, void* host_dst, size_t bytes) {
         case JTP_STAGE_SUMS: {
             if (!c.p.tree_enabled) return fail(&c, JTP_ERR_STATE, "tree disabled");
             std::vector<uint64_t> raw(nI * 8);
+            JTP_HIP(&c, stage_node_sums(c, n, nullptr));
             JTP_HIP(&c, hipMemcpy(raw.data(), c.node_sum, nI * 64, hipMemcpyDeviceToHost));
             uint64_t* o = (uint64_t*)host_dst;
             for (int64_t i = 0; i < nI; ++i) {

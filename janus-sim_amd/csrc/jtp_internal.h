@@ -29,13 +29,11 @@ constexpr int kLightMax = 1024;      // tiles with at most this many are light (
 inline int64_t interp_list_size(int64_t G3, int64_t n) {
     return (G3 / 512 + 1) / 2 + n / kInterpChunk + n / (kLightMax + 1) + 1;
 }
-constexpr int kMaxRounds = 128;      // size of the bottom-up control block (frontier count ... root flag)
 constexpr int kXcds = 8;             // MI355X accelerator complex dies; workgroup i runs on XCD i % 8
 // device counter block (int32): offsets
 constexpr int kCtrNGroups = 0, kCtrErr = 1, kCtrDense = 3, kCtrInterp = 4;  // kCtrInterp: 3 words
-constexpr int kCtrRounds = 8;                       // [0] global frontier size, [kMaxRounds+1] root flag
-constexpr int kCtrRoot = kCtrRounds + kMaxRounds + 1;
-constexpr int kCtrXcd = 192;                        // kXcds walk-queue heads, kCtrXcdStride apart
+constexpr int kCtrRoot = 7;                         // 1: the build completed the root
+constexpr int kCtrXcd = 64;                         // kXcds walk-queue heads, kCtrXcdStride apart
 constexpr int kCtrXcdStride = 64;                   // 256 bytes: their atomics do not share a line
 constexpr int kCtrTotal = kCtrXcd + kXcds * kCtrXcdStride;
 
@@ -149,7 +147,7 @@ struct Ctx {
     // capacities (elements)
     int64_t cap_n = 0;
     // particle-side buffers
-    uint64_t *keys0 = nullptr, *keys1 = nullptr;  // keys1: the sort's second buffer, then the build's int2 leaf ranges
+    uint64_t *keys0 = nullptr, *keys1 = nullptr;  // keys1: the sort's second buffer
     int32_t *vals0 = nullptr, *vals1 = nullptr;
     uint32_t *hist = nullptr;        // 256 * nblocks
     uint32_t *hist_blk = nullptr;    // scan partials
@@ -157,17 +155,15 @@ struct Ctx {
     // tree
     uint4 *node_geo = nullptr;       // 2 per internal node: (centre xyz, first leaf), (extent xyz, last leaf)
     int2 *node_kids = nullptr;
-    int2 *up = nullptr;              // internal node: (parent, sibling); the root's parent is -1
-    int32_t *flags = nullptr;        // bottom-up arrival counters
-    int32_t *frontier0 = nullptr;    // bottom-up: nodes whose range crosses a chunk edge, ready to climb
-    int32_t *frontier1 = nullptr;    // bottom-up: nodes whose range crosses a superchunk edge, ready to climb
+    int32_t *bt_count = nullptr;     // build: unmerged runs of each workgroup's list
     int32_t *dense_list = nullptr;   // deposit: the PM cells holding more than kDenseCell particles
     int2 *interp_list = nullptr;     // FP32 interpolation: the light tiles (G^3 / 512 int32), then the
                                      // (tile, first particle) of the heavy tiles' chunks; interp_list_size
     int2 *dep_chunks = nullptr;      // FP32 deposit: (tile, first particle) of the chunks of tiles holding
                                      // more than kInterpChunk particles; dep_chunk_cap entries
     long long *dep_cbuf = nullptr;   // FP32 deposit: int64 LDS grid of each such chunk (1729 per entry)
-    void *node_sum = nullptr;        // NodeSum per internal node
+    void *node_sum = nullptr;        // 64 bytes per particle: the packed records before the gather, then the build's
+                                     // lists of unmerged runs; NodeSum per node for the stage export
     void *node_mono = nullptr;       // 2 x (uint4 | double4) per internal node
     int2 *groups = nullptr;
     int32_t *cell4 = nullptr;        // level-4 cell offsets (4097)
@@ -250,7 +246,10 @@ hipError_t device_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 hipError_t launch_gather_parts(const uint4* rec, const int32_t* perm, uint4* parts, int64_t n, int32_t* tile_start,
                                int logG, hipStream_t s);
 
-hipError_t build_tree(Ctx& c, int64_t n, hipStream_t s);            // Karras + bottom-up + mono + groups
+hipError_t build_tree(Ctx& c, int64_t n, hipStream_t s);            // radix tree with boxes and monopoles, groups
+hipError_t launch_reset(Ctx& c, hipStream_t s);                     // counters and start cells of an evaluation
+hipError_t stage_node_sums(Ctx& c, int64_t n, hipStream_t s);       // c.node_sum <- NodeSum of every node
+inline int64_t bt_count_size(int64_t cap) { return cap / 256 + 128; }
 hipError_t launch_fill_i32(int32_t* out, int64_t m, int32_t v, hipStream_t s);
 hipError_t launch_cell_start(const uint64_t* keys, int64_t n, int shift, int64_t ncells, int32_t* out,
                              hipStream_t s);
