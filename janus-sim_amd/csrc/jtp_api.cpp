@@ -275,7 +275,7 @@ static int ensure_capacity(Ctx& c, int64_t n) {
     chk(dalloc(c.keys1, cap));
     chk(dalloc(c.vals0, cap));
     chk(dalloc(c.vals1, cap));
-    chk(dalloc(c.hist, m));
+    chk(dalloc(c.hist, std::max(m, sort_hist_size(cap))));
     chk(dalloc(c.hist_blk, (m + 2047) / 2048 + 1));
     chk(dalloc(c.parts, cap));
     chk(dalloc(c.node_geo, 2 * cap));
@@ -522,12 +522,8 @@ static int enqueue_prep(Ctx& c, int64_t n, const uint32_t* d_pos, const int8_t* 
                         bool timed) {
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[0], s));
     JTP_HIP(&c, launch_reset(c, s));
-    // the packed records live in the node-sum buffer, which the tree build (after the gather) overwrites
-    uint4* rec = (uint4*)c.node_sum;
-    JTP_HIP(&c, launch_morton_keys(d_pos, d_species, c.keys0, c.vals0, rec, n, s));
-    JTP_HIP(&c, radix_sort_pairs(c, n, s, kKeyLowBits));
     const bool tiles = c.p.pm_enabled && c.p.precision == JTP_FP32;  // tile starts for the FP32 PM
-    JTP_HIP(&c, launch_gather_parts(rec, c.vals0, c.parts, n, tiles ? c.tile_start : nullptr, c.logG, s));
+    JTP_HIP(&c, sort_particles(c, d_pos, d_species, n, tiles ? c.tile_start : nullptr, s));
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[1], s));
     // The tree build and the PM phases only share read-only inputs (sorted keys and records), so the
     // build runs on the side stream while the PM phases run on `s`; the walk waits for both.

@@ -68,8 +68,7 @@ __host__ __device__ inline uint64_t morton_fixed(uint32_t ux, uint32_t uy, uint3
 // key), so the two radix passes over those bits are skipped.
 constexpr int kKeyLowBits = 16;
 constexpr uint64_t kKeySortMask = ~((1ull << kKeyLowBits) - 1);
-static_assert(kKeyLowBits % 8 == 0 && (64 - kKeyLowBits) / 8 % 2 == 0,
-              "whole 8-bit radix passes, an even number of them (the result lands in the first buffer)");
+static_assert(kKeyLowBits == 16, "the particle sort takes 48 key bits as six 8-bit digits");
 
 // Split-function coefficients for the FP32 walk, rho^2 = r^2 + eps^2, x = rho / (2 r_s):
 //  * particle pairs under erfc + Gaussian (always cut at r_cut): S(x) - 1 = x^3 h(x^2) with h entire,
@@ -149,7 +148,7 @@ struct Ctx {
     // particle-side buffers
     uint64_t *keys0 = nullptr, *keys1 = nullptr;  // keys1: the sort's second buffer
     int32_t *vals0 = nullptr, *vals1 = nullptr;
-    uint32_t *hist = nullptr;        // 256 * nblocks
+    uint32_t *hist = nullptr;        // digit counts of the sorts
     uint32_t *hist_blk = nullptr;    // scan partials
     uint4 *parts = nullptr;          // sorted records: fixed xyz + species
     // tree
@@ -231,21 +230,18 @@ struct Ctx {
 // All return hipError_t from hipGetLastError after the launch(es).
 hipError_t launch_fixed_from_f64(const double* pos, uint32_t* out, int64_t n3, double L, hipStream_t s);
 hipError_t launch_fixed_from_f32(const float* pos, uint32_t* out, int64_t n3, double L, hipStream_t s);
-// keys, identity values and the packed (x, y, z, species) records in input order
-hipError_t launch_morton_keys(const uint32_t* pos, const int8_t* species, uint64_t* keys, int32_t* vals,
-                              uint4* rec, int64_t n, hipStream_t s);
+// The particles in Morton order: c.keys0 (sorted keys), c.vals0 (input indices), c.parts (records); with tile_start (FP32
+// PM), also the first sorted particle of every Morton-aligned 8^3-cell tile of the mesh, tile_start[ntile] = n
+hipError_t sort_particles(Ctx& c, const uint32_t* pos, const int8_t* species, int64_t n, int32_t* tile_start,
+                          hipStream_t s);
+int64_t sort_hist_size(int64_t cap);  // entries of c.hist for that
 hipError_t launch_morton_keys_f32(const float* pos, uint64_t* keys, int64_t n, float box_half,
                                   float inv_cell, hipStream_t s);
 hipError_t launch_morton30_keys_f32(const float* pos, uint64_t* keys, int32_t* idx, int64_t n, float box_half,
                                     hipStream_t s);
-// keys0/vals0 -> keys0/vals0 sorted by the key bits from first_bit (a multiple of 16) up, stable
-hipError_t radix_sort_pairs(Ctx& c, int64_t n, hipStream_t s, int first_bit = 0);
+// keys0/vals0 -> keys0/vals0 sorted by the 64-bit keys, stable
+hipError_t radix_sort_pairs(Ctx& c, int64_t n, hipStream_t s);
 hipError_t device_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
-// parts[i] = rec[perm[i]]; with tile_start (FP32 PM), also the first sorted particle of every
-// Morton-aligned 8^3-cell tile of the 2^logG mesh, tile_start[ntile] = n
-hipError_t launch_gather_parts(const uint4* rec, const int32_t* perm, uint4* parts, int64_t n, int32_t* tile_start,
-                               int logG, hipStream_t s);
-
 hipError_t build_tree(Ctx& c, int64_t n, hipStream_t s);            // radix tree with boxes and monopoles, groups
 hipError_t launch_reset(Ctx& c, hipStream_t s);                     // counters and start cells of an evaluation
 hipError_t stage_node_sums(Ctx& c, int64_t n, hipStream_t s);       // c.node_sum <- NodeSum of every node
