@@ -453,10 +453,6 @@ int jtp_create(const jtp_params* p, jtp_ctx** out) {
     if (e == hipSuccess) e = dalloc(c.diag_scratch, kDiagScratch);
     if (e == hipSuccess) e = hipHostMalloc((void**)&c.host_step, sizeof(StepParams), 0);
     make_split_poly(c);
-    if (p->precision == JTP_FP64) {  // the walk's polynomials
-        if (e == hipSuccess) e = dalloc(c.dev_fit64, 1);
-        if (e == hipSuccess) e = hipMemcpy(c.dev_fit64, &c.poly64, sizeof(SplitPoly64), hipMemcpyHostToDevice);
-    }
     if (e == hipSuccess) e = pm_tables(c);
     if (e == hipSuccess) {
         for (int i = 0; i < 10 && e == hipSuccess; ++i) e = hipEventCreate(&c.ev[i]);
@@ -543,8 +539,7 @@ static int enqueue_prep(Ctx& c, int64_t n, const uint32_t* d_pos, const int8_t* 
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[2], s));
     if (c.p.pm_enabled) JTP_HIP(&c, pm_deposit(c, n, s));
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[3], s));
-    if (c.p.pm_enabled) JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, s));
-    if (c.p.pm_enabled && c.p.interlace) JTP_HIP(&c, pm_fft_solve(c, c.rho2, c.phi2, s));
+    if (c.p.pm_enabled) JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, c.rho2, c.phi2, s));  // rho2: null without interlacing
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[4], s));
     if (c.p.pm_enabled) JTP_HIP(&c, pm_interp(c, n, s));
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[5], s));
@@ -587,7 +582,25 @@ static int check_status(Ctx& c, int64_t n) {
     return JTP_OK;
 }
 
+// What an evaluation needs beyond a mesh solve (contexts that only solve never pay for it): the particle buffers, the half
+// spectrum of the second mesh and the FP64 walk's polynomials.
 static int prepare(Ctx& c, int64_t n) {
+    if (c.p.interlace && !c.spec_pair) {
+        void* two = nullptr;
+        const hipError_t e = hipMalloc(&two, (size_t)c.G() * c.G() * c.Hc() * 4 * c.real_size());
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(&c, JTP_ERR_ALLOC, std::string("device allocation failed: ") + hipGetErrorString(e));
+        }
+        (void)hipFree(c.spec);
+        c.spec = two;
+        c.spec_pair = true;
+        c.graph_dirty = true;
+    }
+    if (c.poly64.ok && !c.dev_fit64) {
+        JTP_HIP(&c, dalloc(c.dev_fit64, 1));
+        JTP_HIP(&c, hipMemcpy(c.dev_fit64, &c.poly64, sizeof(SplitPoly64), hipMemcpyHostToDevice));
+    }
     const int64_t old_cap = c.cap_n;
     int rc = ensure_capacity(c, n);
     if (rc != JTP_OK) return rc;
@@ -840,7 +853,7 @@ int jtp_potential_energy(jtp_ctx* h, int64_t n, const uint32_t* d_pos, const int
         const double one = 1.0;
         JTP_HIP(&c, hipStreamSynchronize(s));
         JTP_HIP(&c, hipMemcpy(c.rho, &one, sizeof(double), hipMemcpyHostToDevice));
-        JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, s, 0));
+        JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, nullptr, nullptr, s, 0));
         JTP_HIP(&c, hipStreamSynchronize(s));
         double k27[27];
         const int64_t G = c.G();
@@ -857,8 +870,7 @@ int jtp_potential_energy(jtp_ctx* h, int64_t n, const uint32_t* d_pos, const int
     // The force's Green function is matched to the gradient stencil, which distorts the potential at
     // a few cells; the energy uses the potential of the plain deconvolved Gaussian-split Green function
     // (the same one the self-energy kernel was computed with).
-    JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, s, 0));
-    if (c.p.interlace) JTP_HIP(&c, pm_fft_solve(c, c.rho2, c.phi2, s, 0));
+    JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, c.rho2, c.phi2, s, 0));
     double* res = c.diag_scratch + 1024 * 8;
     JTP_HIP(&c, launch_energy_terms(c, n, c.kself, c.pot_short, c.diag_scratch, res, s));
     double host[5];
@@ -907,7 +919,7 @@ int jtp_pm_solve(jtp_ctx* h, const void* d_rho, void* d_phi, void* stream) {
     if (!h) return JTP_ERR_ARG;
     if (!d_rho || !d_phi) return fail(&h->c, JTP_ERR_ARG, "null grid pointer");
     hipStream_t s = (hipStream_t)stream;
-    JTP_HIP(&h->c, pm_fft_solve(h->c, d_rho, d_phi, s));
+    JTP_HIP(&h->c, pm_fft_solve(h->c, d_rho, d_phi, nullptr, nullptr, s));
     JTP_HIP(&h->c, hipStreamSynchronize(s));
     return JTP_OK;
 }

@@ -181,7 +181,8 @@ struct Ctx {
     void *rho2 = nullptr, *phi2 = nullptr;  // interlaced grid (nodes at the cell centres of the first)
     void *grad = nullptr, *grad2 = nullptr;  // FP64: real4 [G^3] stencil gradient of phi / phi2 (w unused); FP32: grad
                                              // is allocated only by jtp_generate_ics (one real grid)
-    void *spec = nullptr;            // complex G^2 (G/2+1)
+    void *spec = nullptr;            // complex G^2 (G/2+1); two of them once spec_pair is set
+    bool spec_pair = false;          // interlaced contexts, from the first evaluation on
     void *twiddle = nullptr;         // complex G  e^{-2 pi i m/G}
     void *gtab = nullptr;            // real 2G: per-axis window/Gaussian factor, k_i^2
     void *pm_acc = nullptr;          // real 3n (sorted order)
@@ -256,7 +257,9 @@ int64_t dep_chunk_nodes();         // FP32 deposit: int64 node sums per chunk en
 int64_t dep_tile_record();         // FP32 deposit: floats per tile record (own blocks, beyond nodes)
 // phi <- Green * rho; matched = 1 multiplies by the gradient-stencil match (the force's Green
 // function when deconvolving; -1 = as the context's force), 0 leaves the potential unmatched
-hipError_t pm_fft_solve(Ctx& c, const void* rho, void* phi, hipStream_t s, int matched = -1);
+// and, unless rho2 is null, phi2 <- Green * rho2 in the same launches (contexts with interlacing)
+hipError_t pm_fft_solve(Ctx& c, const void* rho, void* phi, const void* rho2, void* phi2, hipStream_t s,
+                        int matched = -1);
 // out <- unnormalised inverse real 3-D FFT of the Hermitian half spectrum in c.spec (overwritten)
 hipError_t pm_inverse_fft(Ctx& c, void* out, hipStream_t s);
 // Zel'dovich lattice initial conditions of G^3 particles (G = the context's mesh)

@@ -763,10 +763,21 @@ __global__ void k_deposit(const uint4* __restrict__ parts, const int32_t* __rest
 // v_r = x[j + r G/R], multiplies by w^(r k) (k = j mod Ns, w = exp(-+2 pi i / (R Ns)), from the
 // table tw[m] = e^{-2 pi i m / G}), does the R-point DFT and writes y_r to
 // (j / Ns) R Ns + k + r Ns (autosorted order); reads go to registers, a barrier, then the writes.
-template <int LG, int LP, bool LINE_FAST>
+// Where point p of line l lies among the 2^LP points of a workgroup: line by line, point by point, or in a plane
+// (kPlane, below).
+enum FftMap { kLines, kPoints, kPlane };
+// Slot of index i of a line-by-line or plane layout: bits 5-7 and 6-7 are XORed into bits 0-2 and 3-4, so that the
+// strided writes of the first two stages (p = 8 j + r, then 64 (j / 8) + 8 r + j % 8) fall on different banks, as runs of
+// consecutive indices do.  (Unswizzled the first stage's writes take 8 times their cycles.)
+__device__ inline int fft_slot(int i) { return i ^ ((i >> 5) & 7) ^ (((i >> 6) & 3) << 3); }
+template <int LG, int LP, FftMap MAP>
 __device__ inline int fft_at(int l, int p) {
-    constexpr int LNL = LP - LG;  // log2 of the line count (2^LP points per workgroup)
-    return LINE_FAST ? l + (p << LNL) : (l << LG) + p;
+    constexpr int LNL = LP - LG, G = 1 << LG;  // log2 of the line count (2^LP points per workgroup)
+    if constexpr (MAP == kLines) return fft_slot((l << LG) + p);
+    if constexpr (MAP == kPoints) return l + (p << LNL);
+    // column l of row p: the two rows of a pair share G slots, the odd row's columns mirrored
+    const int base = (p >> 1) << LG;
+    return fft_slot((p & 1) == 0 ? base + l : base + (l == 0 ? G / 2 : G - l));
 }
 
 template <typename R>
@@ -831,24 +842,25 @@ __device__ inline void dft_small(const Cplx<R>* v, Cplx<R>* y, bool inv) {
 // One Stockham stage of radix 2^LR after LS bits (Ns = 2^LS): butterfly j reads points
 // j + r G / RAD, multiplies point r by W_{RAD Ns}^{r k} (k = j mod Ns, tw[m] = e^{-2 pi i m / G}),
 // and writes output r to ((j / Ns) RAD Ns + k) + r Ns; all reads, a barrier, all writes.
-template <typename R, int LG, int LP, bool LINE_FAST, int LR, int LS>
+template <typename R, int LG, int LP, FftMap MAP, int LR, int LS, int T>
 __device__ inline void fft_stage(Cplx<R>* buf, const Cplx<R>* tw, bool inv) {
 #pragma clang fp contract(off)
     constexpr int RAD = 1 << LR, G = 1 << LG, LNL = LP - LG, Q = G / RAD, LQ = LG - LR, Ns = 1 << LS;
-    constexpr int NB = (1 << LP) / RAD / 256;  // butterflies per thread
-    static_assert(NB >= 1, "a workgroup holds at least 256 butterflies");
+    constexpr bool FAST = MAP != kLines;       // neighbouring threads take neighbouring lines
+    constexpr int NB = (1 << LP) / RAD / T;    // butterflies per thread
+    static_assert(NB >= 1, "a butterfly per thread at least");
     const int tid = threadIdx.x;
     Cplx<R> y[NB][RAD];
     int ll[NB], oo[NB];
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
-        const int q = tid + u * 256;
-        const int l = LINE_FAST ? (q & ((1 << LNL) - 1)) : (q >> LQ);
-        const int j = LINE_FAST ? (q >> LNL) : (q & (Q - 1));
+        const int q = tid + u * T;
+        const int l = FAST ? (q & ((1 << LNL) - 1)) : (q >> LQ);
+        const int j = FAST ? (q >> LNL) : (q & (Q - 1));
         const int k = j & (Ns - 1);
         Cplx<R> v[RAD];
 #pragma unroll
-        for (int r = 0; r < RAD; ++r) v[r] = buf[fft_at<LG, LP, LINE_FAST>(l, j + r * Q)];
+        for (int r = 0; r < RAD; ++r) v[r] = buf[fft_at<LG, LP, MAP>(l, j + r * Q)];
         if constexpr (LS > 0) {  // the first stage's twiddles are all 1
 #pragma unroll
             for (int r = 1; r < RAD; ++r) {
@@ -865,37 +877,44 @@ __device__ inline void fft_stage(Cplx<R>* buf, const Cplx<R>* tw, bool inv) {
 #pragma unroll
     for (int u = 0; u < NB; ++u)
 #pragma unroll
-        for (int r = 0; r < RAD; ++r) buf[fft_at<LG, LP, LINE_FAST>(ll[u], oo[u] + r * Ns)] = y[u][r];
+        for (int r = 0; r < RAD; ++r) buf[fft_at<LG, LP, MAP>(ll[u], oo[u] + r * Ns)] = y[u][r];
     __syncthreads();
 }
 
 // Radix-8 stages while three or more bits remain, then one radix-4 or radix-2 stage
 // (G = 512: 8 8 8; 256: 8 8 4; 128: 8 8 2; 64: 8 8; 32: 8 4; 16: 8 2).
-template <typename R, int LG, int LP, bool LINE_FAST, int LS>
+template <typename R, int LG, int LP, FftMap MAP, int LS, int T>
 __device__ inline void fft_stages(Cplx<R>* buf, const Cplx<R>* tw, bool inv) {
     if constexpr (LG - LS >= 3) {
-        fft_stage<R, LG, LP, LINE_FAST, 3, LS>(buf, tw, inv);
-        fft_stages<R, LG, LP, LINE_FAST, LS + 3>(buf, tw, inv);
+        fft_stage<R, LG, LP, MAP, 3, LS, T>(buf, tw, inv);
+        fft_stages<R, LG, LP, MAP, LS + 3, T>(buf, tw, inv);
     } else if constexpr (LG - LS == 2) {
-        fft_stage<R, LG, LP, LINE_FAST, 2, LS>(buf, tw, inv);
+        fft_stage<R, LG, LP, MAP, 2, LS, T>(buf, tw, inv);
     } else if constexpr (LG - LS == 1) {
-        fft_stage<R, LG, LP, LINE_FAST, 1, LS>(buf, tw, inv);
+        fft_stage<R, LG, LP, MAP, 1, LS, T>(buf, tw, inv);
     }
 }
 
-// 2^LP / G lines of G points in LDS (LINE_FAST: point p of line l at l + p 2^(LP-LG), else l G + p),
-// transformed in place; no FMA contraction, so every tile size rounds each butterfly identically.
-template <typename R, int LG, int LP, bool LINE_FAST>
+// 2^LP / G lines of G points in LDS (fft_at), transformed in place by T threads; no FMA contraction, so every tile
+// size rounds each butterfly identically.
+template <typename R, int LG, int LP, FftMap MAP, int T = 256>
 __device__ inline void lds_fft(Cplx<R>* buf, const Cplx<R>* __restrict__ tw, bool inv) {
-    static_assert(LP >= 11 && LP >= LG, "one radix-8 butterfly per thread and one line per block");
-    fft_stages<R, LG, LP, LINE_FAST, 0>(buf, tw, inv);
+    static_assert(LP >= LG && (1 << LP) / 8 >= T, "one radix-8 butterfly per thread and one line per block");
+    fft_stages<R, LG, LP, MAP, 0, T>(buf, tw, inv);
 }
+
+// The real meshes of one launch: blockIdx.y = 0 or 1 (the two interlaced ones), and their half spectra one after the
+// other.
+template <typename R> struct MeshPair { R *a, *b; };
+__host__ __device__ constexpr int64_t spec_size(int64_t G) { return G * G * (G / 2 + 1); }
 
 // X forward (R2C): pairs of real lines (y even, y odd) packed as one complex line.
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_x_r2c(const R* __restrict__ in, Cplx<R>* __restrict__ out,
+__global__ __launch_bounds__(256) void k_fft_x_r2c(MeshPair<const R> real, Cplx<R>* __restrict__ spec,
                                                    const Cplx<R>* __restrict__ tw) {
 #pragma clang fp contract(off)
+    const R* __restrict__ in = blockIdx.y ? real.b : real.a;
+    Cplx<R>* __restrict__ out = spec + blockIdx.y * spec_size(1 << LG);
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
@@ -917,20 +936,20 @@ __global__ __launch_bounds__(256) void k_fft_x_r2c(const R* __restrict__ in, Cpl
 #pragma unroll
             for (int i = 0; i < VW; ++i) v[i] = (R)0;
         }
-        Cplx<R>* b = &buf[(line >> 1) * G + x];
 #pragma unroll
         for (int i = 0; i < VW; ++i) {
-            if (line & 1) b[i].y = v[i]; else b[i].x = v[i];
+            Cplx<R>& b = buf[fft_slot((line >> 1) * G + x + i)];
+            if (line & 1) b.y = v[i]; else b.x = v[i];
         }
     }
     __syncthreads();
-    lds_fft<R, LG, LP, false>(buf, stw, false);
+    lds_fft<R, LG, LP, kLines>(buf, stw, false);
     Cplx<R>* dst = out + line0 * H;
     for (int e = threadIdx.x; e < rows * H; e += 256) {
         const int row = e / H, k = e - row * H;
         const int p = row >> 1;
-        const Cplx<R> z = buf[p * G + k];
-        const Cplx<R> zc = buf[p * G + ((G - k) & (G - 1))];
+        const Cplx<R> z = buf[fft_slot(p * G + k)];
+        const Cplx<R> zc = buf[fft_slot(p * G + ((G - k) & (G - 1)))];
         Cplx<R> o;
         if ((row & 1) == 0) {  // A = (Z[k] + conj Z[G-k]) / 2
             o = {(R)0.5 * (z.x + zc.x), (R)0.5 * (z.y - zc.y)};
@@ -943,8 +962,10 @@ __global__ __launch_bounds__(256) void k_fft_x_r2c(const R* __restrict__ in, Cpl
 
 // X inverse (C2R): two half-spectrum rows A, B -> Z = A + i B, inverse FFT, re / im = the two real rows.
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_x_c2r(const Cplx<R>* __restrict__ in, R* __restrict__ out,
+__global__ __launch_bounds__(256) void k_fft_x_c2r(const Cplx<R>* __restrict__ spec, MeshPair<R> real,
                                                    const Cplx<R>* __restrict__ tw) {
+    R* __restrict__ out = blockIdx.y ? real.b : real.a;
+    const Cplx<R>* __restrict__ in = spec + blockIdx.y * spec_size(1 << LG);
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
@@ -966,59 +987,82 @@ __global__ __launch_bounds__(256) void k_fft_x_c2r(const Cplx<R>* __restrict__ i
             a.y = 0;
             b.y = 0;
         }
-        buf[p * G + k] = {a.x - b.y, a.y + b.x};
-        if (k > 0 && k < G / 2) buf[p * G + G - k] = {a.x + b.y, -a.y + b.x};  // conj A + i conj B
+        buf[fft_slot(p * G + k)] = {a.x - b.y, a.y + b.x};
+        if (k > 0 && k < G / 2) buf[fft_slot(p * G + G - k)] = {a.x + b.y, -a.y + b.x};  // conj A + i conj B
     }
     __syncthreads();
-    lds_fft<R, LG, LP, false>(buf, stw, true);
+    lds_fft<R, LG, LP, kLines>(buf, stw, true);
     R* dst = out + line0 * G;
     constexpr int VW = 16 / (int)sizeof(R);  // 16-byte stores of VW consecutive x
     for (int e4 = threadIdx.x; e4 < rows * G / VW; e4 += 256) {
         const int e = e4 * VW, line = e >> LG, x = e & (G - 1);
-        const Cplx<R>* z = &buf[(line >> 1) * G + x];
         R v[VW];
 #pragma unroll
-        for (int i = 0; i < VW; ++i) v[i] = (line & 1) ? z[i].y : z[i].x;
+        for (int i = 0; i < VW; ++i) {
+            const Cplx<R> z = buf[fft_slot((line >> 1) * G + x + i)];
+            v[i] = (line & 1) ? z.y : z.x;
+        }
         uint4 w;
         __builtin_memcpy(&w, v, 16);
         *(uint4*)(dst + e) = w;
     }
 }
 
-// Block -> (plane, kx block) for the y and z passes.  A workgroup reads KB consecutive kx of every
-// row, i.e. KB * sizeof(complex) bytes per row (64 B at G = 512 in FP32: half a 128-byte line),
-// and the other half of each line belongs to the next kx block.  Blocks are dispatched round-robin
-// over the 8 XCDs, so consecutive logical blocks are dealt to one XCD in sequence: the kx block
-// that reads the other half of the lines runs next on the same XCD and finds them in its L2.
+// The lines of the y and z passes, numbered through: line q of the z pass is (ky, kx) = (q / H, q % H) and starts at q; of
+// the y pass (z, kx), starting at z G H + kx.  A workgroup takes KB consecutive lines, so no lane is spent on the part of a
+// kx block beyond H (with blocks of kx per row 5 % of the lines at G = 256, 19 % in FP64 at 128, 73 % at 32).  It reads
+// KB * sizeof(complex) bytes per row (64 B at G = 512 in FP32: half a 128-byte line), and the other half of each line
+// belongs to the next block.  Blocks are dispatched round-robin over the 8 XCDs, so consecutive logical blocks are dealt
+// to one XCD in sequence: the block that reads the other half of the lines runs next on the same XCD and finds them in
+// its L2.
 __device__ inline int fft_logical_block(int nblocks) {
     const int b = (int)blockIdx.x;
     return (nblocks & 7) ? b : (b & 7) * (nblocks >> 3) + (b >> 3);
 }
+template <int LG, int LP> constexpr int fft_blocks() { return (int)((spec_size(1 << LG) + (1 << LP) - 1) >> LP); }
 
-// Y pass (complex, forward or inverse): block = (z, block of KB consecutive kx).
+// One workgroup's lines of the y or z pass: the thread's line, its start and the distance of its points; the thread's
+// elements are points tid / KB, tid / KB + 256 / KB, ... of it.
+template <int LG, int LP, bool Z>
+struct FftLines {
+    static constexpr int G = 1 << LG, H = G / 2 + 1, KB = 1 << (LP - LG), LKB = LP - LG;
+    static_assert(KB <= 256, "a thread stays on its line");
+    bool in;
+    int a, kx;  // ky (z pass) or z (y pass), and kx
+    int64_t start;
+    static constexpr int64_t stride = Z ? (int64_t)G * H : H;
+    __device__ FftLines() {
+        const int lb = fft_logical_block(fft_blocks<LG, LP>());
+        const int q = lb * KB + (int)(threadIdx.x & (KB - 1));
+        in = q < G * H;
+        a = q / H;
+        kx = q - a * H;
+        start = Z ? (int64_t)q : (int64_t)a * (G * H) + kx;
+    }
+    template <typename R>
+    __device__ void load(const Cplx<R>* __restrict__ spec, Cplx<R>* buf) const {
+        for (int e = threadIdx.x; e < (1 << LP); e += 256)
+            buf[e] = in ? spec[start + (e >> LKB) * stride] : Cplx<R>{0, 0};
+    }
+    template <typename R>
+    __device__ void store(Cplx<R>* __restrict__ spec, const Cplx<R>* buf) const {
+        if (!in) return;
+        for (int e = threadIdx.x; e < (1 << LP); e += 256) spec[start + (e >> LKB) * stride] = buf[e];
+    }
+};
+
+// Y pass (complex, forward or inverse).
 template <typename R, int LG, int LP>
 __global__ __launch_bounds__(256) void k_fft_y(Cplx<R>* __restrict__ spec, const Cplx<R>* __restrict__ tw, int inv) {
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
-    constexpr int G = 1 << LG, H = G / 2 + 1;
-    constexpr int KB = (1 << LP) / G, LKB = LP - LG;
-    constexpr int nkb = (H + KB - 1) / KB;
-    const int lb = fft_logical_block(G * nkb);
-    const int z = lb / nkb, kx0 = (lb % nkb) * KB;
-    Cplx<R>* base = spec + (int64_t)z * G * H;
-    for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int y = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
-        buf[e] = (kx < H) ? base[(int64_t)y * H + kx] : Cplx<R>{0, 0};
-    }
+    spec += blockIdx.y * spec_size(1 << LG);
+    const FftLines<LG, LP, false> ln;
+    ln.load(spec, buf);
     __syncthreads();
-    lds_fft<R, LG, LP, true>(buf, stw, inv != 0);
-    for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int y = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
-        if (kx < H) base[(int64_t)y * H + kx] = buf[e];
-    }
+    lds_fft<R, LG, LP, kPoints>(buf, stw, inv != 0);
+    ln.store(spec, buf);
 }
 
 // Z pass with the Green function: forward z FFT, multiply, inverse z FFT.
@@ -1030,48 +1074,37 @@ __global__ __launch_bounds__(256) void k_fft_z_green(Cplx<R>* __restrict__ spec,
 #pragma clang fp contract(off)
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
-    for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
-    constexpr int G = 1 << LG, H = G / 2 + 1;
-    constexpr int KB = (1 << LP) / G, LKB = LP - LG;
-    constexpr int nkb = (H + KB - 1) / KB;
-    const int lb = fft_logical_block(G * nkb);
-    const int y = lb / nkb, kx0 = (lb % nkb) * KB;
-    constexpr int64_t zs = (int64_t)G * H;
-    Cplx<R>* base = spec + (int64_t)y * H;
-    for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int z = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
-        buf[e] = (kx < H) ? base[z * zs + kx] : Cplx<R>{0, 0};
-    }
+    constexpr int G = 1 << LG;
+    constexpr bool kTab = LG <= 7;    // small meshes: also the Green tables, read beside the lines
+    __shared__ R stab[kTab ? 4 << LG : 1];
+    for (int i = threadIdx.x; i < G; i += 256) stw[i] = tw[i];
+    if (kTab)
+        for (int i = threadIdx.x; i < 4 * G; i += 256) stab[i] = gtab[i];
+    spec += blockIdx.y * spec_size(G);
+    using Lines = FftLines<LG, LP, true>;
+    const Lines ln;
+    ln.load(spec, buf);
     __syncthreads();
-    lds_fft<R, LG, LP, true>(buf, stw, false);
-    const R* T = gtab;
-    const R* K2 = gtab + G;
-    const R* Ks = gtab + 2 * G;  // signed k_i
-    const R* D = gtab + 3 * G;   // transfer function of the gradient stencil along one axis
-    const int ky = y;
+    lds_fft<R, LG, LP, kPoints>(buf, stw, false);
+    const R* T = kTab ? stab : gtab;
+    const R* K2 = T + G;
+    const R* Ks = T + 2 * G;  // signed k_i
+    const R* D = T + 3 * G;   // transfer function of the gradient stencil along one axis
+    const int ky = ln.in ? ln.a : 0, kx = ln.kx;  // the thread's line
     const int aky = ky <= G / 2 ? ky : G - ky;
-    const R Ty = T[ky], K2y = K2[ky], Ksy = Ks[ky], Dy = D[ky];  // the block's row: one ky
-    // with KB <= 256 every element of a thread has the same kx (256 is a multiple of KB)
-    const int kx_t = kx0 + (threadIdx.x & (KB - 1));
-    const int kx_c = kx_t < H ? kx_t : 0;
-    const R Tx_t = T[kx_c], K2x_t = K2[kx_c], Ksx_t = Ks[kx_c], Dx_t = D[kx_c];
+    const R Ty = T[ky], K2y = K2[ky], Ksy = Ks[ky], Dy = D[ky];
+    const R Tx = T[kx], K2x = K2[kx], Ksx = Ks[kx], Dx = D[kx];
     for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int kz = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
+        const int kz = e >> Lines::LKB;
         const int akz = kz <= G / 2 ? kz : G - kz;
-        const int akx = kx;
-        const int kmax = max(akx, max(aky, akz));
+        const int kmax = max(kx, max(aky, akz));
         R f = 0;
-        if (kx < H && !(akx == 0 && aky == 0 && akz == 0) && kmax >= k_min) {
-            const bool same = KB <= 256;
-            const R Tx = same ? Tx_t : T[kx], K2x = same ? K2x_t : K2[kx];
+        if (!(kx == 0 && aky == 0 && akz == 0) && kmax >= k_min) {
             const R k2 = K2x + K2y + K2[kz];
             f = norm * Tx * Ty * T[kz];
             if (matched) {
                 // least-squares match of the stencil gradient D to i k: f *= (k . D) / |D|^2, with the
                 // denominator floored at |k|^2 / 4 where D vanishes (Nyquist planes); one division
-                const R Ksx = same ? Ksx_t : Ks[kx], Dx = same ? Dx_t : D[kx];
                 const R dd = Dx * Dx + Dy * Dy + D[kz] * D[kz];
                 const R fl = (R)0.25 * k2;
                 f = f * (Ksx * Dx + Ksy * Dy + Ks[kz] * D[kz]) / (k2 * (dd > fl ? dd : fl));
@@ -1083,12 +1116,8 @@ __global__ __launch_bounds__(256) void k_fft_z_green(Cplx<R>* __restrict__ spec,
         buf[e] = {v.x * f, v.y * f};
     }
     __syncthreads();
-    lds_fft<R, LG, LP, true>(buf, stw, true);
-    for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int z = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
-        if (kx < H) base[z * zs + kx] = buf[e];
-    }
+    lds_fft<R, LG, LP, kPoints>(buf, stw, true);
+    ln.store(spec, buf);
 }
 
 // Inverse z pass alone (the z pass of the solver without the forward transform and Green multiply).
@@ -1097,31 +1126,143 @@ __global__ __launch_bounds__(256) void k_fft_z_inv(Cplx<R>* __restrict__ spec, c
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
-    constexpr int G = 1 << LG, H = G / 2 + 1;
-    constexpr int KB = (1 << LP) / G, LKB = LP - LG;
-    constexpr int nkb = (H + KB - 1) / KB;
-    const int lb = fft_logical_block(G * nkb);
-    const int y = lb / nkb, kx0 = (lb % nkb) * KB;
-    constexpr int64_t zs = (int64_t)G * H;
-    Cplx<R>* base = spec + (int64_t)y * H;
-    for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int z = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
-        buf[e] = (kx < H) ? base[z * zs + kx] : Cplx<R>{0, 0};
+    const FftLines<LG, LP, true> ln;
+    ln.load(spec, buf);
+    __syncthreads();
+    lds_fft<R, LG, LP, kPoints>(buf, stw, true);
+    ln.store(spec, buf);
+}
+
+// ---- meshes whose xy planes fit the LDS (G = 32, 64, 128): x and y in one pass each way.
+//
+// A plane of G x G reals is G / 2 packed complex lines.  After the x transforms the half spectra A, B of the two rows
+// of a line are unpacked in place, pair by pair: slots k and G - k hold Z[k] and Z[G - k] before, A[k] and B[k] after
+// (kPlane); slots 0 and G / 2 then hold (A[0], A[G/2]) and (B[0], B[G/2]), all real, so column 0 carries the columns 0 and
+// G / 2 as one complex sequence that is taken apart after the y transform.  T threads, a radix-8 butterfly each.
+//
+// Three launches a solve instead of five, and the half spectrum moved 4 times instead of 8; such meshes are bound by the
+// launches and each workgroup's chain of LDS stages (one mesh of 128 planes fills half the CUs).  Measured, with both
+// interlaced meshes in the same launches, ms: 0.056 -> 0.025 at G = 32, 0.08 -> 0.033 at 64, 0.126 -> 0.070 at 128 (FP32);
+// one FP64 mesh at 128 with its call 0.077 -> 0.072.
+template <int LG> constexpr int plane_threads() { return LG == 7 ? 1024 : (LG == 6 ? 256 : 64); }
+
+template <typename R, int LG>
+__global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R> real, Cplx<R>* __restrict__ spec,
+                                                                const Cplx<R>* __restrict__ tw) {
+#pragma clang fp contract(off)
+    constexpr int G = 1 << LG, H = G / 2 + 1, LP = 2 * LG - 1, T = plane_threads<LG>();
+    __shared__ Cplx<R> buf[1 << LP];
+    __shared__ Cplx<R> stw[G];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < G; i += T) stw[i] = tw[i];
+    const R* __restrict__ src = (blockIdx.y ? real.b : real.a) + (int64_t)blockIdx.x * G * G;
+    constexpr int VW = 16 / (int)sizeof(R);  // 16-byte loads of consecutive x
+#pragma unroll 4
+    for (int e4 = tid; e4 < G * G / VW; e4 += T) {
+        const int e = e4 * VW, row = e >> LG, x = e & (G - 1);
+        const uint4 w = *(const uint4*)(src + e);
+        R v[VW];
+        __builtin_memcpy(v, &w, 16);
+#pragma unroll
+        for (int i = 0; i < VW; ++i) {
+            Cplx<R>& b = buf[fft_slot(((row >> 1) << LG) + x + i)];
+            if (row & 1) b.y = v[i]; else b.x = v[i];
+        }
     }
     __syncthreads();
-    lds_fft<R, LG, LP, true>(buf, stw, true);
-    for (int e = threadIdx.x; e < (1 << LP); e += 256) {
-        const int z = e >> LKB, jb = e & (KB - 1);
-        const int kx = kx0 + jb;
-        if (kx < H) base[z * zs + kx] = buf[e];
+    lds_fft<R, LG, LP, kLines, T>(buf, stw, false);
+#pragma unroll 4
+    for (int e = tid; e < G * G / 4; e += T) {
+        const int p = e >> (LG - 1), k = e & (G / 2 - 1);
+        Cplx<R>& u = buf[fft_slot((p << LG) + k)];
+        Cplx<R>& w = buf[fft_slot((p << LG) + (k == 0 ? G / 2 : G - k))];
+        const Cplx<R> z = u, zc = w;
+        if (k == 0) {
+            u = {z.x, zc.x};
+            w = {z.y, zc.y};
+        } else {
+            u = {(R)0.5 * (z.x + zc.x), (R)0.5 * (z.y - zc.y)};  // A = (Z[k] + conj Z[G-k]) / 2
+            w = {(R)0.5 * (z.y + zc.y), (R)0.5 * (zc.x - z.x)};  // B = (Z[k] - conj Z[G-k]) / (2i)
+        }
+    }
+    __syncthreads();
+    lds_fft<R, LG, LP, kPlane, T>(buf, stw, false);
+    Cplx<R>* __restrict__ dst = spec + blockIdx.y * spec_size(G) + (int64_t)blockIdx.x * G * H;
+    for (int e = tid; e < G * H; e += T) {
+        const int r = e / H, k = e - r * H;
+        Cplx<R> o = buf[fft_at<LG, LP, kPlane>(k & (G / 2 - 1), r)];
+        if ((k & (G / 2 - 1)) == 0) {
+            const Cplx<R> n = buf[fft_at<LG, LP, kPlane>(0, (G - r) & (G - 1))];
+            o = k == 0 ? Cplx<R>{(R)0.5 * (o.x + n.x), (R)0.5 * (o.y - n.y)}
+                       : Cplx<R>{(R)0.5 * (o.y + n.y), (R)0.5 * (n.x - o.x)};
+        }
+        dst[e] = o;
+    }
+}
+
+template <typename R, int LG>
+__global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(const Cplx<R>* __restrict__ spec, MeshPair<R> real,
+                                                                const Cplx<R>* __restrict__ tw) {
+#pragma clang fp contract(off)
+    constexpr int G = 1 << LG, H = G / 2 + 1, LP = 2 * LG - 1, T = plane_threads<LG>();
+    __shared__ Cplx<R> buf[1 << LP];
+    __shared__ Cplx<R> stw[G];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < G; i += T) stw[i] = tw[i];
+    const Cplx<R>* __restrict__ src = spec + blockIdx.y * spec_size(G) + (int64_t)blockIdx.x * G * H;
+#pragma unroll 4
+    for (int e = tid; e < G * G / 2; e += T) {
+        const int r = e >> (LG - 1), k = e & (G / 2 - 1);
+        Cplx<R> v = src[r * H + k];
+        if (k == 0) {
+            // columns 0 and G / 2 become real in the y transform: their Hermitian parts, packed
+            const int n = (G - r) & (G - 1);
+            const Cplx<R> w = src[n * H], x = src[r * H + G / 2], y = src[n * H + G / 2];
+            const Cplx<R> f = {(R)0.5 * (v.x + w.x), (R)0.5 * (v.y - w.y)};
+            const Cplx<R> g = {(R)0.5 * (x.x + y.x), (R)0.5 * (x.y - y.y)};
+            v = {f.x - g.y, f.y + g.x};
+        }
+        buf[fft_at<LG, LP, kPlane>(k, r)] = v;
+    }
+    __syncthreads();
+    lds_fft<R, LG, LP, kPlane, T>(buf, stw, true);
+#pragma unroll 4
+    for (int e = tid; e < G * G / 4; e += T) {
+        const int p = e >> (LG - 1), k = e & (G / 2 - 1);
+        Cplx<R>& u = buf[fft_slot((p << LG) + k)];
+        Cplx<R>& w = buf[fft_slot((p << LG) + (k == 0 ? G / 2 : G - k))];
+        const Cplx<R> a = u, b = w;
+        if (k == 0) {
+            u = {a.x, b.x};
+            w = {a.y, b.y};
+        } else {
+            u = {a.x - b.y, a.y + b.x};   // A + i B
+            w = {a.x + b.y, -a.y + b.x};  // conj A + i conj B
+        }
+    }
+    __syncthreads();
+    lds_fft<R, LG, LP, kLines, T>(buf, stw, true);
+    R* __restrict__ dst = (blockIdx.y ? real.b : real.a) + (int64_t)blockIdx.x * G * G;
+    constexpr int VW = 16 / (int)sizeof(R);
+#pragma unroll 4
+    for (int e4 = tid; e4 < G * G / VW; e4 += T) {
+        const int e = e4 * VW, row = e >> LG, x = e & (G - 1);
+        R v[VW];
+#pragma unroll
+        for (int i = 0; i < VW; ++i) {
+            const Cplx<R> z = buf[fft_slot(((row >> 1) << LG) + x + i)];
+            v[i] = (row & 1) ? z.y : z.x;
+        }
+        uint4 w;
+        __builtin_memcpy(&w, v, 16);
+        *(uint4*)(dst + e) = w;
     }
 }
 
 // One Poisson solve's device buffers and constants: the context's, or the scratch of the
 // allocation-free entry point.
 struct FftPlan {
-    void* spec;           // half spectrum, complex [G][G][G/2+1]
+    void* spec;           // half spectrum, complex [G][G][G/2+1], one per mesh of a solve
     const void* twiddle;  // complex [G]
     const void* gtab;     // real [4 G]: T, k^2, k, stencil transfer D per axis index
     double green_norm;
@@ -1132,39 +1273,54 @@ static FftPlan plan_of(const Ctx& c) {
     return FftPlan{c.spec, c.twiddle, c.gtab, c.green_norm, c.logG, c.p.k_min, c.p.fft_tile, c.p.precision};
 }
 
+template <int LG> constexpr bool plane_fits() { return LG >= 5 && LG <= 7; }
+
 template <typename R, int LG, int LP>
 static hipError_t inverse_fft_lg(const FftPlan& f, R* out, hipStream_t s) {
-    constexpr int G = 1 << LG, H = G / 2 + 1, NPT = 1 << LP;
-    constexpr int KB = NPT / G, nkb = (H + KB - 1) / KB;
+    constexpr int G = 1 << LG, NPT = 1 << LP;
     constexpr unsigned nx = (unsigned)(G * G > 2 * (NPT / G) ? (int64_t)G * G / (2 * (NPT / G)) : 1);
     const Cplx<R>* tw = (const Cplx<R>*)f.twiddle;
     Cplx<R>* spec = (Cplx<R>*)f.spec;
-    k_fft_z_inv<R, LG, LP><<<dim3((unsigned)(G * nkb)), dim3(256), 0, s>>>(spec, tw);
-    k_fft_y<R, LG, LP><<<dim3((unsigned)(G * nkb)), dim3(256), 0, s>>>(spec, tw, 1);
-    k_fft_x_c2r<R, LG, LP><<<dim3(nx), dim3(256), 0, s>>>(spec, out, tw);
+    const MeshPair<R> o{out, nullptr};
+    k_fft_z_inv<R, LG, LP><<<dim3(fft_blocks<LG, LP>()), dim3(256), 0, s>>>(spec, tw);
+    if constexpr (plane_fits<LG>()) {
+        k_fft_yx<R, LG><<<dim3(G), dim3(plane_threads<LG>()), 0, s>>>(spec, o, tw);
+    } else {
+        k_fft_y<R, LG, LP><<<dim3(fft_blocks<LG, LP>()), dim3(256), 0, s>>>(spec, tw, 1);
+        k_fft_x_c2r<R, LG, LP><<<dim3(nx), dim3(256), 0, s>>>(spec, o, tw);
+    }
     return hipGetLastError();
 }
 
+// `nm` meshes (1, or the 2 interlaced ones) in the same launches.
 template <typename R, int LG, int LP>
-static hipError_t fft_solve_lg(const FftPlan& f, const R* rho, R* phi, hipStream_t s, int matched) {
-    constexpr int G = 1 << LG, H = G / 2 + 1, NPT = 1 << LP;
-    constexpr int KB = NPT / G, nkb = (H + KB - 1) / KB;
+static hipError_t fft_solve_lg(const FftPlan& f, MeshPair<const R> rho, MeshPair<R> phi, unsigned nm, hipStream_t s,
+                               int matched) {
+    constexpr int G = 1 << LG, NPT = 1 << LP, nb = fft_blocks<LG, LP>();
     constexpr unsigned nx = (unsigned)(G * G > 2 * (NPT / G) ? (int64_t)G * G / (2 * (NPT / G)) : 1);
     const Cplx<R>* tw = (const Cplx<R>*)f.twiddle;
     Cplx<R>* spec = (Cplx<R>*)f.spec;
-    k_fft_x_r2c<R, LG, LP><<<dim3(nx), dim3(256), 0, s>>>(rho, spec, tw);
-    k_fft_y<R, LG, LP><<<dim3((unsigned)(G * nkb)), dim3(256), 0, s>>>(spec, tw, 0);
-    k_fft_z_green<R, LG, LP><<<dim3((unsigned)(G * nkb)), dim3(256), 0, s>>>(spec, tw, (const R*)f.gtab,
-                                                                         (R)f.green_norm, f.k_min, matched);
-    k_fft_y<R, LG, LP><<<dim3((unsigned)(G * nkb)), dim3(256), 0, s>>>(spec, tw, 1);
-    k_fft_x_c2r<R, LG, LP><<<dim3(nx), dim3(256), 0, s>>>(spec, phi, tw);
+    if constexpr (plane_fits<LG>()) {
+        k_fft_xy<R, LG><<<dim3(G, nm), dim3(plane_threads<LG>()), 0, s>>>(rho, spec, tw);
+    } else {
+        k_fft_x_r2c<R, LG, LP><<<dim3(nx, nm), dim3(256), 0, s>>>(rho, spec, tw);
+        k_fft_y<R, LG, LP><<<dim3(nb, nm), dim3(256), 0, s>>>(spec, tw, 0);
+    }
+    k_fft_z_green<R, LG, LP><<<dim3(nb, nm), dim3(256), 0, s>>>(spec, tw, (const R*)f.gtab, (R)f.green_norm, f.k_min,
+                                                               matched);
+    if constexpr (plane_fits<LG>()) {
+        k_fft_yx<R, LG><<<dim3(G, nm), dim3(plane_threads<LG>()), 0, s>>>(spec, phi, tw);
+    } else {
+        k_fft_y<R, LG, LP><<<dim3(nb, nm), dim3(256), 0, s>>>(spec, tw, 1);
+        k_fft_x_c2r<R, LG, LP><<<dim3(nx, nm), dim3(256), 0, s>>>(spec, phi, tw);
+    }
     return hipGetLastError();
 }
 
 // the mesh sizes the context accepts (G = 16 .. 512) and FFT tiles (2^11, 2^12 points; 2^13 for FP32)
 #define JTP_FFT_DISPATCH_LG(CALL, LP)          \
     switch (f.logG) {                          \
-        case 4: return CALL(4, LP);            \
+        case 4: return CALL(4, (LP < 12 ? LP : 12)); /* at most 256 lines of 16 points */ \
         case 5: return CALL(5, LP);            \
         case 6: return CALL(6, LP);            \
         case 7: return CALL(7, LP);            \
@@ -1191,8 +1347,9 @@ hipError_t pm_inverse_fft(Ctx& c, void* out, hipStream_t s) {
 }
 
 template <typename R>
-static hipError_t fft_solve_t(const FftPlan& f, const R* rho, R* phi, hipStream_t s, int matched) {
-#define JTP_SOLVE(LG, LP) fft_solve_lg<R, LG, LP>(f, rho, phi, s, matched)
+static hipError_t fft_solve_t(const FftPlan& f, MeshPair<const R> rho, MeshPair<R> phi, unsigned nm, hipStream_t s,
+                              int matched) {
+#define JTP_SOLVE(LG, LP) fft_solve_lg<R, LG, LP>(f, rho, phi, nm, s, matched)
     if constexpr (sizeof(R) == 4) {
         if (f.tile == 13) JTP_FFT_DISPATCH_LG(JTP_SOLVE, 13)
     }
@@ -1201,14 +1358,21 @@ static hipError_t fft_solve_t(const FftPlan& f, const R* rho, R* phi, hipStream_
 #undef JTP_SOLVE
 }
 
-static hipError_t plan_solve(const FftPlan& f, const void* rho, void* phi, hipStream_t s, int matched) {
-    if (f.precision == JTP_FP64) return fft_solve_t<double>(f, (const double*)rho, (double*)phi, s, matched);
-    return fft_solve_t<float>(f, (const float*)rho, (float*)phi, s, matched);
+template <typename R>
+static hipError_t plan_solve_t(const FftPlan& f, const void* rho, void* phi, const void* rho2, void* phi2,
+                               hipStream_t s, int matched) {
+    return fft_solve_t<R>(f, MeshPair<const R>{(const R*)rho, (const R*)rho2}, MeshPair<R>{(R*)phi, (R*)phi2},
+                          rho2 ? 2u : 1u, s, matched);
+}
+static hipError_t plan_solve(const FftPlan& f, const void* rho, void* phi, const void* rho2, void* phi2, hipStream_t s,
+                             int matched) {
+    if (f.precision == JTP_FP64) return plan_solve_t<double>(f, rho, phi, rho2, phi2, s, matched);
+    return plan_solve_t<float>(f, rho, phi, rho2, phi2, s, matched);
 }
 
-hipError_t pm_fft_solve(Ctx& c, const void* rho, void* phi, hipStream_t s, int matched) {
+hipError_t pm_fft_solve(Ctx& c, const void* rho, void* phi, const void* rho2, void* phi2, hipStream_t s, int matched) {
     if (matched < 0) matched = c.p.deconvolve;  // the force's Green function
-    return plan_solve(plan_of(c), rho, phi, s, matched);
+    return plan_solve(plan_of(c), rho, phi, rho2, phi2, s, matched);
 }
 
 // deposit chunks of tiles holding more than kInterpChunk particles: sum over those tiles of
@@ -1824,6 +1988,6 @@ extern "C" int jtp_pm_solve_noalloc(const jtp_params* p, const void* d_rho, void
         k_pm_tables<float><<<dim3((G + 127) / 128), dim3(128), 0, s>>>((float*)f.twiddle, (float*)f.gtab, G,
                                                                        p->box_size, p->r_s, p->deconvolve, four);
     if (hipGetLastError() != hipSuccess) return JTP_ERR_HIP;
-    if (plan_solve(f, d_rho, d_phi, s, p->deconvolve) != hipSuccess) return JTP_ERR_HIP;
+    if (plan_solve(f, d_rho, d_phi, nullptr, nullptr, s, p->deconvolve) != hipSuccess) return JTP_ERR_HIP;
     return JTP_OK;
 }

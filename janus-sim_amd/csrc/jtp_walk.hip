@@ -784,7 +784,7 @@ static void fill_args(Ctx& c, int64_t n, void* acc_out, WalkArgs& a) {
     a.qp = c.p.g_constant * c.m_plus;
     a.qm = -c.p.g_constant * c.m_minus;
     a.poly = c.poly;
-    a.fit64 = c.poly64.ok ? c.dev_fit64 : nullptr;
+    a.fit64 = c.dev_fit64;  // set where poly64.ok
     // t = x * 2/X - 1 with x = rho/(2 r_s) and X the fit range (make_split_poly)
     a.tscale = c.poly_tscale;
     a.tscale_m = c.poly_tscale_m;
