@@ -479,7 +479,7 @@ int jtp_destroy(jtp_ctx* h) {
     free_particle_buffers(c);
     if (c.graph.exec) (void)hipGraphExecDestroy(c.graph.exec);
     if (c.graph.capture_stream) (void)hipStreamDestroy(c.graph.capture_stream);
-    void* ptrs[] = {c.rho, c.phi, c.rho2, c.phi2, c.grad, c.grad2, c.spec, c.twiddle, c.gtab, c.cell_start,
+    void* ptrs[] = {c.rho, c.phi, c.rho2, c.phi2, c.grad, c.grad2, c.spec, c.spec2, c.twiddle, c.gtab, c.cell_start,
                     c.tile_start, c.dep_tbuf,
                     c.cell4, c.cellnode, c.dev_counters, c.dev_inter, c.dense_slot, c.dev_step, c.diag_scratch,
                     c.pot_short, c.acc_scratch, c.kself, c.seg, c.dev_fit64};
@@ -585,17 +585,12 @@ static int check_status(Ctx& c, int64_t n) {
 // What an evaluation needs beyond a mesh solve (contexts that only solve never pay for it): the particle buffers, the half
 // spectrum of the second mesh and the FP64 walk's polynomials.
 static int prepare(Ctx& c, int64_t n) {
-    if (c.p.interlace && !c.spec_pair) {
-        void* two = nullptr;
-        const hipError_t e = hipMalloc(&two, (size_t)c.G() * c.G() * c.Hc() * 4 * c.real_size());
+    if (c.p.interlace && c.p.pm_enabled && !c.spec2) {
+        const hipError_t e = dalloc_bytes(c.spec2, (size_t)c.G() * c.G() * c.Hc() * 2 * c.real_size());
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return fail(&c, JTP_ERR_ALLOC, std::string("device allocation failed: ") + hipGetErrorString(e));
         }
-        (void)hipFree(c.spec);
-        c.spec = two;
-        c.spec_pair = true;
-        c.graph_dirty = true;
     }
     if (c.poly64.ok && !c.dev_fit64) {
         JTP_HIP(&c, dalloc(c.dev_fit64, 1));

@@ -181,8 +181,8 @@ struct Ctx {
     void *rho2 = nullptr, *phi2 = nullptr;  // interlaced grid (nodes at the cell centres of the first)
     void *grad = nullptr, *grad2 = nullptr;  // FP64: real4 [G^3] stencil gradient of phi / phi2 (w unused); FP32: grad
                                              // is allocated only by jtp_generate_ics (one real grid)
-    void *spec = nullptr;            // complex G^2 (G/2+1); two of them once spec_pair is set
-    bool spec_pair = false;          // interlaced contexts, from the first evaluation on
+    void *spec = nullptr;            // complex G^2 (G/2+1)
+    void *spec2 = nullptr;           // the second mesh's; interlaced contexts, from the first evaluation on
     void *twiddle = nullptr;         // complex G  e^{-2 pi i m/G}
     void *gtab = nullptr;            // real 2G: per-axis window/Gaussian factor, k_i^2
     void *pm_acc = nullptr;          // real 3n (sorted order)

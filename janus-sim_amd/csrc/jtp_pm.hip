@@ -903,18 +903,20 @@ __device__ inline void lds_fft(Cplx<R>* buf, const Cplx<R>* __restrict__ tw, boo
     fft_stages<R, LG, LP, MAP, 0, T>(buf, tw, inv);
 }
 
-// The real meshes of one launch: blockIdx.y = 0 or 1 (the two interlaced ones), and their half spectra one after the
-// other.
-template <typename R> struct MeshPair { R *a, *b; };
+// The meshes of one launch, or their half spectra: blockIdx.y = 0 or 1 (the two interlaced ones).
+template <typename R> struct MeshPair {
+    R *a, *b;
+    __device__ R* mine() const { return blockIdx.y ? b : a; }
+};
 __host__ __device__ constexpr int64_t spec_size(int64_t G) { return G * G * (G / 2 + 1); }
 
 // X forward (R2C): pairs of real lines (y even, y odd) packed as one complex line.
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_x_r2c(MeshPair<const R> real, Cplx<R>* __restrict__ spec,
+__global__ __launch_bounds__(256) void k_fft_x_r2c(MeshPair<const R> real, MeshPair<Cplx<R>> spec,
                                                    const Cplx<R>* __restrict__ tw) {
 #pragma clang fp contract(off)
-    const R* __restrict__ in = blockIdx.y ? real.b : real.a;
-    Cplx<R>* __restrict__ out = spec + blockIdx.y * spec_size(1 << LG);
+    const R* __restrict__ in = real.mine();
+    Cplx<R>* __restrict__ out = spec.mine();
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
@@ -962,10 +964,10 @@ __global__ __launch_bounds__(256) void k_fft_x_r2c(MeshPair<const R> real, Cplx<
 
 // X inverse (C2R): two half-spectrum rows A, B -> Z = A + i B, inverse FFT, re / im = the two real rows.
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_x_c2r(const Cplx<R>* __restrict__ spec, MeshPair<R> real,
+__global__ __launch_bounds__(256) void k_fft_x_c2r(MeshPair<Cplx<R>> spec, MeshPair<R> real,
                                                    const Cplx<R>* __restrict__ tw) {
-    R* __restrict__ out = blockIdx.y ? real.b : real.a;
-    const Cplx<R>* __restrict__ in = spec + blockIdx.y * spec_size(1 << LG);
+    R* __restrict__ out = real.mine();
+    const Cplx<R>* __restrict__ in = spec.mine();
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
@@ -1053,11 +1055,11 @@ struct FftLines {
 
 // Y pass (complex, forward or inverse).
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_y(Cplx<R>* __restrict__ spec, const Cplx<R>* __restrict__ tw, int inv) {
+__global__ __launch_bounds__(256) void k_fft_y(MeshPair<Cplx<R>> pair, const Cplx<R>* __restrict__ tw, int inv) {
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
-    spec += blockIdx.y * spec_size(1 << LG);
+    Cplx<R>* __restrict__ spec = pair.mine();
     const FftLines<LG, LP, false> ln;
     ln.load(spec, buf);
     __syncthreads();
@@ -1069,7 +1071,7 @@ __global__ __launch_bounds__(256) void k_fft_y(Cplx<R>* __restrict__ spec, const
 // green(kx, ky, kz) = norm * T[kx] T[ky] T[kz] / (K2[kx] + K2[ky] + K2[kz]); zero for DC and
 // for max(|kx|,|ky|,|kz|) < k_min (apply_green_kernel, cufft_wrapper.cu:160-207).
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_z_green(Cplx<R>* __restrict__ spec, const Cplx<R>* __restrict__ tw,
+__global__ __launch_bounds__(256) void k_fft_z_green(MeshPair<Cplx<R>> pair, const Cplx<R>* __restrict__ tw,
                                                      const R* __restrict__ gtab, R norm, int k_min, int matched) {
 #pragma clang fp contract(off)
     __shared__ Cplx<R> buf[1 << LP];
@@ -1080,7 +1082,7 @@ __global__ __launch_bounds__(256) void k_fft_z_green(Cplx<R>* __restrict__ spec,
     for (int i = threadIdx.x; i < G; i += 256) stw[i] = tw[i];
     if (kTab)
         for (int i = threadIdx.x; i < 4 * G; i += 256) stab[i] = gtab[i];
-    spec += blockIdx.y * spec_size(G);
+    Cplx<R>* __restrict__ spec = pair.mine();
     using Lines = FftLines<LG, LP, true>;
     const Lines ln;
     ln.load(spec, buf);
@@ -1122,10 +1124,11 @@ __global__ __launch_bounds__(256) void k_fft_z_green(Cplx<R>* __restrict__ spec,
 
 // Inverse z pass alone (the z pass of the solver without the forward transform and Green multiply).
 template <typename R, int LG, int LP>
-__global__ __launch_bounds__(256) void k_fft_z_inv(Cplx<R>* __restrict__ spec, const Cplx<R>* __restrict__ tw) {
+__global__ __launch_bounds__(256) void k_fft_z_inv(MeshPair<Cplx<R>> pair, const Cplx<R>* __restrict__ tw) {
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[1 << LG];  // the twiddles, staged once (ordered by the barrier after the load)
     for (int i = threadIdx.x; i < (1 << LG); i += 256) stw[i] = tw[i];
+    Cplx<R>* __restrict__ spec = pair.mine();
     const FftLines<LG, LP, true> ln;
     ln.load(spec, buf);
     __syncthreads();
@@ -1147,7 +1150,7 @@ __global__ __launch_bounds__(256) void k_fft_z_inv(Cplx<R>* __restrict__ spec, c
 template <int LG> constexpr int plane_threads() { return LG == 7 ? 1024 : (LG == 6 ? 256 : 64); }
 
 template <typename R, int LG>
-__global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R> real, Cplx<R>* __restrict__ spec,
+__global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R> real, MeshPair<Cplx<R>> spec,
                                                                 const Cplx<R>* __restrict__ tw) {
 #pragma clang fp contract(off)
     constexpr int G = 1 << LG, H = G / 2 + 1, LP = 2 * LG - 1, T = plane_threads<LG>();
@@ -1155,7 +1158,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R
     __shared__ Cplx<R> stw[G];
     const int tid = threadIdx.x;
     for (int i = tid; i < G; i += T) stw[i] = tw[i];
-    const R* __restrict__ src = (blockIdx.y ? real.b : real.a) + (int64_t)blockIdx.x * G * G;
+    const R* __restrict__ src = real.mine() + (int64_t)blockIdx.x * G * G;
     constexpr int VW = 16 / (int)sizeof(R);  // 16-byte loads of consecutive x
 #pragma unroll 4
     for (int e4 = tid; e4 < G * G / VW; e4 += T) {
@@ -1187,7 +1190,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R
     }
     __syncthreads();
     lds_fft<R, LG, LP, kPlane, T>(buf, stw, false);
-    Cplx<R>* __restrict__ dst = spec + blockIdx.y * spec_size(G) + (int64_t)blockIdx.x * G * H;
+    Cplx<R>* __restrict__ dst = spec.mine() + (int64_t)blockIdx.x * G * H;
     for (int e = tid; e < G * H; e += T) {
         const int r = e / H, k = e - r * H;
         Cplx<R> o = buf[fft_at<LG, LP, kPlane>(k & (G / 2 - 1), r)];
@@ -1201,7 +1204,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R
 }
 
 template <typename R, int LG>
-__global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(const Cplx<R>* __restrict__ spec, MeshPair<R> real,
+__global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(MeshPair<Cplx<R>> spec, MeshPair<R> real,
                                                                 const Cplx<R>* __restrict__ tw) {
 #pragma clang fp contract(off)
     constexpr int G = 1 << LG, H = G / 2 + 1, LP = 2 * LG - 1, T = plane_threads<LG>();
@@ -1209,7 +1212,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(const Cplx<R>* _
     __shared__ Cplx<R> stw[G];
     const int tid = threadIdx.x;
     for (int i = tid; i < G; i += T) stw[i] = tw[i];
-    const Cplx<R>* __restrict__ src = spec + blockIdx.y * spec_size(G) + (int64_t)blockIdx.x * G * H;
+    const Cplx<R>* __restrict__ src = spec.mine() + (int64_t)blockIdx.x * G * H;
 #pragma unroll 4
     for (int e = tid; e < G * G / 2; e += T) {
         const int r = e >> (LG - 1), k = e & (G / 2 - 1);
@@ -1242,7 +1245,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(const Cplx<R>* _
     }
     __syncthreads();
     lds_fft<R, LG, LP, kLines, T>(buf, stw, true);
-    R* __restrict__ dst = (blockIdx.y ? real.b : real.a) + (int64_t)blockIdx.x * G * G;
+    R* __restrict__ dst = real.mine() + (int64_t)blockIdx.x * G * G;
     constexpr int VW = 16 / (int)sizeof(R);
 #pragma unroll 4
     for (int e4 = tid; e4 < G * G / VW; e4 += T) {
@@ -1262,7 +1265,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(const Cplx<R>* _
 // One Poisson solve's device buffers and constants: the context's, or the scratch of the
 // allocation-free entry point.
 struct FftPlan {
-    void* spec;           // half spectrum, complex [G][G][G/2+1], one per mesh of a solve
+    void *spec, *spec2;   // half spectra, complex [G][G][G/2+1]; spec2 for a second mesh
     const void* twiddle;  // complex [G]
     const void* gtab;     // real [4 G]: T, k^2, k, stencil transfer D per axis index
     double green_norm;
@@ -1270,7 +1273,7 @@ struct FftPlan {
 };
 
 static FftPlan plan_of(const Ctx& c) {
-    return FftPlan{c.spec, c.twiddle, c.gtab, c.green_norm, c.logG, c.p.k_min, c.p.fft_tile, c.p.precision};
+    return FftPlan{c.spec, c.spec2, c.twiddle, c.gtab, c.green_norm, c.logG, c.p.k_min, c.p.fft_tile, c.p.precision};
 }
 
 template <int LG> constexpr bool plane_fits() { return LG >= 5 && LG <= 7; }
@@ -1280,7 +1283,7 @@ static hipError_t inverse_fft_lg(const FftPlan& f, R* out, hipStream_t s) {
     constexpr int G = 1 << LG, NPT = 1 << LP;
     constexpr unsigned nx = (unsigned)(G * G > 2 * (NPT / G) ? (int64_t)G * G / (2 * (NPT / G)) : 1);
     const Cplx<R>* tw = (const Cplx<R>*)f.twiddle;
-    Cplx<R>* spec = (Cplx<R>*)f.spec;
+    const MeshPair<Cplx<R>> spec{(Cplx<R>*)f.spec, (Cplx<R>*)f.spec2};
     const MeshPair<R> o{out, nullptr};
     k_fft_z_inv<R, LG, LP><<<dim3(fft_blocks<LG, LP>()), dim3(256), 0, s>>>(spec, tw);
     if constexpr (plane_fits<LG>()) {
@@ -1299,7 +1302,7 @@ static hipError_t fft_solve_lg(const FftPlan& f, MeshPair<const R> rho, MeshPair
     constexpr int G = 1 << LG, NPT = 1 << LP, nb = fft_blocks<LG, LP>();
     constexpr unsigned nx = (unsigned)(G * G > 2 * (NPT / G) ? (int64_t)G * G / (2 * (NPT / G)) : 1);
     const Cplx<R>* tw = (const Cplx<R>*)f.twiddle;
-    Cplx<R>* spec = (Cplx<R>*)f.spec;
+    const MeshPair<Cplx<R>> spec{(Cplx<R>*)f.spec, (Cplx<R>*)f.spec2};
     if constexpr (plane_fits<LG>()) {
         k_fft_xy<R, LG><<<dim3(G, nm), dim3(plane_threads<LG>()), 0, s>>>(rho, spec, tw);
     } else {
@@ -1978,7 +1981,7 @@ extern "C" int jtp_pm_solve_noalloc(const jtp_params* p, const void* d_rho, void
     const int G = p->n_cells;
     int logG = 0;
     while ((1 << logG) < G) ++logG;
-    const FftPlan f{b, b + kNoAllocTwOff, b + kNoAllocTabOff, green_norm_of(*p), logG, p->k_min, p->fft_tile,
+    const FftPlan f{b, nullptr, b + kNoAllocTwOff, b + kNoAllocTabOff, green_norm_of(*p), logG, p->k_min, p->fft_tile,
                     p->precision};
     const int four = p->gradient == JTP_GRAD_4PT;
     if (p->precision == JTP_FP64)
