@@ -238,7 +238,7 @@ void make_split_poly(Ctx& c) {
 
 static void free_particle_buffers(Ctx& c) {
     void* ptrs[] = {c.keys0, c.keys1, c.vals0, c.vals1, c.hist, c.hist_blk, c.parts, c.node_geo, c.node_kids,
-                    c.node_sum, c.node_mono, c.groups, c.pm_acc, c.bt_count, c.dense_list, c.dense_corner, c.interp_list, c.dep_chunks,
+                    c.node_sum, c.node_mono, c.groups, c.early, c.pm_acc, c.bt_count, c.dense_list, c.dense_corner, c.interp_list, c.dep_chunks,
                     c.dep_cbuf};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -256,6 +256,7 @@ static void free_particle_buffers(Ctx& c) {
     c.dep_cbuf = nullptr;
     c.node_sum = c.node_mono = nullptr;
     c.groups = nullptr;
+    c.early = nullptr;
     c.pm_acc = nullptr;
     c.cap_n = 0;
 }
@@ -292,6 +293,7 @@ static int ensure_capacity(Ctx& c, int64_t n) {
     chk(dalloc_bytes(c.node_sum, (size_t)cap * 64));
     chk(dalloc_bytes(c.node_mono, (size_t)cap * (rs == 8 ? 64 : 32)));
     chk(dalloc(c.groups, cap + 4096 + 64));
+    chk(dalloc(c.early, (size_t)early_cap(cap)));
     chk(dalloc_bytes(c.pm_acc, (size_t)cap * 3 * rs));
     if (e != hipSuccess) {
         free_particle_buffers(c);

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <cstddef>
 #include <string>
@@ -31,11 +32,16 @@ inline int64_t interp_list_size(int64_t G3, int64_t n) {
 }
 constexpr int kXcds = 8;             // MI355X accelerator complex dies; workgroup i runs on XCD i % 8
 // device counter block (int32): offsets
-constexpr int kCtrNGroups = 0, kCtrErr = 1, kCtrDense = 3, kCtrInterp = 4;  // kCtrInterp: 3 words
+constexpr int kCtrNGroups = 0, kCtrErr = 1, kCtrEarly = 2, kCtrDense = 3, kCtrInterp = 4;  // kCtrInterp: 3 words
 constexpr int kCtrRoot = 7;                         // 1: the build completed the root
 constexpr int kCtrXcd = 64;                         // kXcds walk-queue heads, kCtrXcdStride apart
 constexpr int kCtrXcdStride = 64;                   // 256 bytes: their atomics do not share a line
 constexpr int kCtrTotal = kCtrXcd + kXcds * kCtrXcdStride;
+// Walk groups whose smallest enclosing Morton cell holds more than kEarlySpan times the group's particles are walked
+// first (k_groups); groups[g].y carries the mark.
+constexpr int kEarlySpan = 64;
+constexpr int32_t kEarlyMark = 1 << 30;
+inline int64_t early_cap(int64_t cap) { return cap / 256 + 4096; }  // entries of the list (beyond it: no mark)
 
 // ---------------------------------------------------------------- small types
 template <typename R> struct Cplx { R x, y; };
@@ -164,7 +170,8 @@ struct Ctx {
     void *node_sum = nullptr;        // 64 bytes per particle: the packed records before the gather, then the build's
                                      // lists of unmerged runs; NodeSum per node for the stage export
     void *node_mono = nullptr;       // 2 x (uint4 | double4) per internal node
-    int2 *groups = nullptr;
+    int2 *groups = nullptr;          // first sorted particle, count (| kEarlyMark)
+    int32_t *early = nullptr;        // the marked groups, in any order
     int32_t *cell4 = nullptr;        // level-4 cell offsets (4097)
     int32_t *cellnode = nullptr;     // node holding each Morton cell of level start_level (<= 4096)
     int start_level = 4;             // finest level whose cell edge L / 2^level is >= r_cut (2..4)

@@ -44,6 +44,8 @@ struct WalkArgs {
     const int2* kids;
     const void* mono;
     const int2* groups;
+    const int32_t* early;  // groups to walk first, early_max at most
+    int32_t early_max;
     int32_t* counters;  // kCtr* layout: group count, error flag, per-XCD queue heads
     unsigned long long* inter;
     const void* pm_acc;  // sorted order, nullptr when the PM part is disabled
@@ -56,7 +58,7 @@ struct WalkArgs {
     const int32_t* cellnode;  // node of each Morton cell of level start_level (nullptr: start at the root)
     int32_t start_level;
     double theta_cut2;  // theta_cut^2 for nodes whose box reaches beyond r_cut
-    int64_t max_steps;
+    int32_t max_steps;
     double scale;   // length per fixed-point unit, L / 2^32
     double eps2;
     double rcut2;
@@ -320,10 +322,10 @@ struct WalkLds {
     uint32_t owner[64];  // bucket-particle owner lanes, one round at a time
 };
 
-// One group g of one box: traversal, list evaluation and the output write.  Adds the group's
+// One group gr (first particle, count) of one box: traversal, list evaluation and the output write.  Adds the group's
 // interaction counts to my_inter / my_mono (lane 0's copies are the wavefront's).
 template <typename R, int MODE, int LPT, bool POT, bool FIT>
-__device__ __forceinline__ void walk_group(const WalkArgs& a, int g, WalkLds<R, LPT>& lds, unsigned long long& my_inter,
+__device__ __forceinline__ void walk_group(const WalkArgs& a, int2 gr, WalkLds<R, LPT>& lds, unsigned long long& my_inter,
                                            unsigned long long& my_mono) {
     constexpr int GL = 64 / LPT;  // targets per wavefront
     using E = typename EntryT<R>::T;
@@ -346,7 +348,7 @@ __device__ __forceinline__ void walk_group(const WalkArgs& a, int g, WalkLds<R, 
     while ((1 << app_shift) < a.leaf) ++app_shift;
     const uint64_t lt = lanemask_lt();
 
-    const int2 gr = a.groups[g];
+    gr.y &= kEarlyMark - 1;
     const int tgt = lane % GL, sub = lane / GL;
     const bool valid = tgt < gr.y;
     const int64_t ti = (int64_t)gr.x + (valid ? tgt : 0);
@@ -373,7 +375,7 @@ __device__ __forceinline__ void walk_group(const WalkArgs& a, int g, WalkLds<R, 
     int sp = 1, lp = 0, lm = 0;
     int pidx = -1, pdst = 0;  // a bucket particle to list in the next step (index, list slot)
     int mono_inside = 0;  // monopole entries placed on the particle side since the last flush
-    int64_t steps = 0;
+    int32_t steps_left = a.max_steps;
     if (a.cellnode) {
         // seed with the 27 cells around the group's cell: a cell's edge is >= r_cut, so every
         // source within r_cut of the group lies in them (the group lies inside one cell)
@@ -466,7 +468,7 @@ __device__ __forceinline__ void walk_group(const WalkArgs& a, int g, WalkLds<R, 
     };
 
     while (sp > 0) {
-        if (++steps > a.max_steps) {  // a finite hierarchy never gets here; report instead of spinning
+        if (--steps_left < 0) {  // a finite hierarchy never gets here; report instead of spinning
             if (lane == 0) atomicExch(&a.counters[kCtrErr], 2);
             break;
         }
@@ -630,18 +632,21 @@ __device__ __forceinline__ void walk_group(const WalkArgs& a, int g, WalkLds<R, 
 // The heads lie 256 bytes apart and a wave that finds nothing leaves with one read: with the heads in
 // one line and an atomic per empty range, the waves' ends cost 0.09 ms of every launch (0.28 ms with the
 // group count in that line too).
-__device__ inline int next_item(int32_t n_items, int32_t* heads, int xcd) {
+// Of n_first + n_items items the first n_first are cut into ranges of their own; a range's are taken before its others.
+__device__ inline int next_item(int32_t n_first, int32_t n_items, int32_t* heads, int xcd) {
     const int lane = threadIdx.x & 63;
     const int q0 = (lane + xcd) % kXcds;  // lane l < 8 looks after the l-th range in this workgroup's order
-    const int32_t start = (int32_t)((int64_t)n_items * q0 / kXcds);
-    const int32_t count = (int32_t)((int64_t)n_items * (q0 + 1) / kXcds) - start;
+    const int32_t start = (int32_t)((int64_t)n_items * q0 / kXcds), fstart = (int32_t)((int64_t)n_first * q0 / kXcds);
+    const int32_t fcount = (int32_t)((int64_t)n_first * (q0 + 1) / kXcds) - fstart;
+    const int32_t count = (int32_t)((int64_t)n_items * (q0 + 1) / kXcds) - start + fcount;
     int pick = 0;  // the own range first, without a look at the heads
     while (true) {
         int t = 0;
         if (lane == pick) t = atomicAdd(&heads[q0 * kCtrXcdStride], 1);
         const bool got = lane == pick && t < count;
         const uint64_t m = __ballot(got);
-        if (m) return __builtin_amdgcn_readlane(start + t, __builtin_amdgcn_readfirstlane(pick));
+        if (m) return __builtin_amdgcn_readlane(t < fcount ? fstart + t : n_first + start + t - fcount,
+                                                __builtin_amdgcn_readfirstlane(pick));
         const int32_t head = lane < kXcds ? __hip_atomic_load(&heads[q0 * kCtrXcdStride], __ATOMIC_RELAXED,
                                                               __HIP_MEMORY_SCOPE_AGENT)
                                           : 0;
@@ -658,9 +663,12 @@ __global__ __launch_bounds__(64 * WAVES) void k_walk(WalkArgs a) {
     WalkLds<R, LPT>& lds = lds_s[threadIdx.x >> 6];
     unsigned long long my_inter = 0, my_mono = 0;
     const int32_t n_groups = a.counters[kCtrNGroups];
-    const int xcd = blockIdx.x % kXcds;
-    for (int g; (g = next_item(n_groups, a.counters + kCtrXcd, xcd)) >= 0;)
-        walk_group<R, MODE, LPT, POT, FIT>(a, g, lds, my_inter, my_mono);
+    const int32_t n_early = min(a.counters[kCtrEarly], a.early_max);  // the groups that may be long (k_groups) first
+    for (int t; (t = next_item(n_early, n_groups, a.counters + kCtrXcd, blockIdx.x % kXcds)) >= 0;) {
+        const int2 gr = a.groups[t < n_early ? a.early[t] : t - n_early];
+        if (t >= n_early && (gr.y & kEarlyMark)) continue;
+        walk_group<R, MODE, LPT, POT, FIT>(a, gr, lds, my_inter, my_mono);
+    }
     if ((threadIdx.x & 63) == 0 && my_inter) {
         atomicAdd(a.inter, my_inter);
         atomicAdd(a.inter + 1, my_mono);
@@ -678,7 +686,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_walk_boxes(const WalkArgs* __res
     WalkLds<R, LPT>& lds = lds_s[threadIdx.x >> 6];
     const int32_t n_items = goff[nbox];
     const int xcd = blockIdx.x % kXcds;
-    for (int t; (t = next_item(n_items, heads, xcd)) >= 0;) {
+    for (int t; (t = next_item(0, n_items, heads, xcd)) >= 0;) {
         int lo = 0, hi = nbox;  // largest b with goff[b] <= t
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
@@ -687,7 +695,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_walk_boxes(const WalkArgs* __res
         const int b = __builtin_amdgcn_readfirstlane(lo);
         const WalkArgs& a = boxes[b];
         unsigned long long my_inter = 0, my_mono = 0;
-        walk_group<R, MODE, LPT, false, FIT>(a, t - goff[b], lds, my_inter, my_mono);
+        walk_group<R, MODE, LPT, false, FIT>(a, a.groups[t - goff[b]], lds, my_inter, my_mono);
         if ((threadIdx.x & 63) == 0 && my_inter) {
             atomicAdd(a.inter, my_inter);
             atomicAdd(a.inter + 1, my_mono);
@@ -761,6 +769,8 @@ static void fill_args(Ctx& c, int64_t n, void* acc_out, WalkArgs& a) {
     a.kids = c.node_kids;
     a.mono = c.node_mono;
     a.groups = c.groups;
+    a.early = c.early;
+    a.early_max = (int32_t)early_cap(c.cap_n);
     a.counters = c.dev_counters;
     a.inter = c.dev_inter;
     a.pm_acc = c.p.pm_enabled ? c.pm_acc : nullptr;
@@ -771,7 +781,7 @@ static void fill_args(Ctx& c, int64_t n, void* acc_out, WalkArgs& a) {
     a.leaf = c.p.leaf_size;
     a.cellnode = n >= 2 ? c.cellnode : nullptr;
     a.start_level = c.start_level;
-    a.max_steps = 4 * n + 1024;  // each step pops >= 1 of the <= 2n-1 nodes
+    a.max_steps = (int32_t)std::min<int64_t>(4 * n + 1024, INT32_MAX);  // each step pops >= 1 of the <= 2n-1 nodes
     const double tc = c.p.theta_cut < c.p.theta ? c.p.theta_cut : c.p.theta;
     a.theta_cut2 = tc * tc;
     a.scale = c.p.box_size / 4294967296.0;
