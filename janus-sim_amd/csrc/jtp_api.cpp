@@ -521,7 +521,8 @@ static int enqueue_prep(Ctx& c, int64_t n, const uint32_t* d_pos, const int8_t* 
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[0], s));
     JTP_HIP(&c, launch_reset(c, s));
     const bool tiles = c.p.pm_enabled && c.p.precision == JTP_FP32;  // tile starts for the FP32 PM
-    JTP_HIP(&c, sort_particles(c, d_pos, d_species, n, tiles ? c.tile_start : nullptr, s));
+    JTP_HIP(&c, sort_particles(c, d_pos, d_species, n, tiles ? c.tile_start : nullptr,
+                               c.p.tree_enabled ? c.cell4 : nullptr, s));
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[1], s));
     // The tree build and the PM phases only share read-only inputs (sorted keys and records), so the
     // build runs on the side stream while the PM phases run on `s`; the walk waits for both.

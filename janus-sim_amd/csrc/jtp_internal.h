@@ -239,9 +239,10 @@ struct Ctx {
 hipError_t launch_fixed_from_f64(const double* pos, uint32_t* out, int64_t n3, double L, hipStream_t s);
 hipError_t launch_fixed_from_f32(const float* pos, uint32_t* out, int64_t n3, double L, hipStream_t s);
 // The particles in Morton order: c.keys0 (sorted keys), c.vals0 (input indices), c.parts (records); with tile_start (FP32
-// PM), also the first sorted particle of every Morton-aligned 8^3-cell tile of the mesh, tile_start[ntile] = n
+// PM), also the first sorted particle of every Morton-aligned 8^3-cell tile of the mesh, tile_start[ntile] = n; with cells
+// that of every level kGroupLevelBits cell that holds any
 hipError_t sort_particles(Ctx& c, const uint32_t* pos, const int8_t* species, int64_t n, int32_t* tile_start,
-                          hipStream_t s);
+                          int32_t* cells, hipStream_t s);
 int64_t sort_hist_size(int64_t cap);  // entries of c.hist for that
 hipError_t launch_morton_keys_f32(const float* pos, uint64_t* keys, int64_t n, float box_half,
                                   float inv_cell, hipStream_t s);

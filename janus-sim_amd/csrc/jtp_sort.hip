@@ -682,20 +682,24 @@ __global__ __launch_bounds__(256) void k_part_scatter(const uint32_t* __restrict
 // ---- gather
 // parts[i] = (x, y, z, species) of the i-th particle in key order (reorder_by_idx_*, nbody_gpu_twopass.rs:1490-1514, fused
 // into one 16-byte record), its key and its input index.  With ts, also the start of every Morton-aligned tile of 8^3 PM
-// cells (lt = log2 G - 3 tile bits per axis; the tile index is a prefix of the key): the particle that begins a run
-// writes the starts of the tiles up to its own, so every entry is written once, ts[ntile] = n.  Lanes read the previous
-// particle's tile from their neighbour; lane 0 gathers it again.  SEG: records in segment order with the input index
-// beside the species, workgroups dealt so that each XCD gathers a contiguous part.
+// cells (lt = log2 G - 3 tile bits per axis; the tile index is a prefix of the key), and with cells that of every level
+// kGroupLevelBits cell that holds any (the walk's groups; a search of the keys for them took 20 us at 2e4 particles and
+// 44 beside other boxes' work): the particle that begins a run of tiles writes the starts of the tiles up to its own, so
+// every entry is written once, ts[ntile] = n.  Lanes read the previous particle's tile from their neighbour; lane 0
+// gathers it again.  SEG: records in segment order with the input index beside the species, workgroups dealt so that each
+// XCD gathers a contiguous part.
 template <bool SEG>
 __global__ __launch_bounds__(256) void k_gather_parts(const uint4* __restrict__ rec, const uint32_t* __restrict__ idx,
                                                       uint4* __restrict__ parts, uint64_t* __restrict__ keys,
                                                       int32_t* __restrict__ perm, int64_t n, int32_t* __restrict__ ts,
-                                                      int lt) {
+                                                      int lt, int32_t* __restrict__ cells) {
     int64_t blk = blockIdx.x;
     if (SEG) blk = (int64_t)(blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
     const int64_t i = blk * blockDim.x + threadIdx.x;
     const bool in = i < n;
-    uint4 r = make_uint4(0u, 0u, 0u, 0u);
+    const bool edge = (threadIdx.x & 63) == 0 && i > 0 && in && (ts || cells);
+    uint4 r = make_uint4(0u, 0u, 0u, 0u), before = r;
+    if (edge) before = rec[idx[i - 1]];
     if (in) {
         const uint32_t k = idx[i];
         r = rec[k];
@@ -704,15 +708,21 @@ __global__ __launch_bounds__(256) void k_gather_parts(const uint4* __restrict__ 
         parts[i] = r;
         keys[i] = morton_fixed(r.x, r.y, r.z) & kKeySortMask;
     }
+    auto tile_of = [&](const uint4& q, int sh) {
+        return (int32_t)(spread3_21(q.x >> sh) | (spread3_21(q.y >> sh) << 1) | (spread3_21(q.z >> sh) << 2));
+    };
+    if (cells) {
+        const int32_t c = in ? tile_of(r, 32 - kGroupLevelBits) : -1;
+        int32_t cp = __shfl_up(c, 1, 64);
+        if ((threadIdx.x & 63) == 0) cp = edge ? tile_of(before, 32 - kGroupLevelBits) : -1;
+        if (in && c != cp) cells[c] = (int32_t)i;
+    }
     if (!ts) return;
     const int sh = 32 - lt;
     const int32_t ntile = 1 << (3 * lt);
-    auto tile_of = [&](const uint4& q) {
-        return (int32_t)(spread3_21(q.x >> sh) | (spread3_21(q.y >> sh) << 1) | (spread3_21(q.z >> sh) << 2));
-    };
-    const int32_t tc = in ? tile_of(r) : ntile;
+    const int32_t tc = in ? tile_of(r, sh) : ntile;
     int32_t tp = __shfl_up(tc, 1, 64);
-    if ((threadIdx.x & 63) == 0) tp = (i == 0 || !in) ? -1 : tile_of(rec[idx[i - 1]]);
+    if ((threadIdx.x & 63) == 0) tp = edge ? tile_of(before, sh) : -1;
     if (!in) return;
     for (int32_t t = tp + 1; t <= tc; ++t) ts[t] = (int32_t)i;
     if (i == n - 1)
@@ -787,7 +797,8 @@ static void sort_segments(Ctx& c, const uint32_t* pos, const int8_t* species, ui
 // partition's tiles.
 int64_t sort_hist_size(int64_t cap) { return (cap / (256 * kSmallIpt) + kSegs + 1) * 256 + kSegs; }
 
-hipError_t sort_particles(Ctx& c, const uint32_t* pos, const int8_t* species, int64_t n, int32_t* ts, hipStream_t s) {
+hipError_t sort_particles(Ctx& c, const uint32_t* pos, const int8_t* species, int64_t n, int32_t* ts, int32_t* cells,
+                          hipStream_t s) {
     if (n <= 0) {
         if (!ts) return hipGetLastError();
         return launch_fill_i32(ts, ((int64_t)1 << (3 * (c.logG - 3))) + 1, 0, s);
@@ -798,13 +809,13 @@ hipError_t sort_particles(Ctx& c, const uint32_t* pos, const int8_t* species, in
     const int lt = c.logG - 3;
     if (n <= (int64_t)kSmallTiles * 256 * kSmallIpt) {
         sort_small<kSmallIpt>(c, pos, species, rec, n, s);
-        k_gather_parts<false><<<dim3(nb), dim3(kBlock), 0, s>>>(rec, idx, c.parts, c.keys0, c.vals0, n, ts, lt);
+        k_gather_parts<false><<<dim3(nb), dim3(kBlock), 0, s>>>(rec, idx, c.parts, c.keys0, c.vals0, n, ts, lt, cells);
     } else {
         // tiles of 6144 once there are enough for the CUs: longer runs per digit
         if (n < (int64_t)4 << 20) sort_segments<kSmallIpt>(c, pos, species, rec, n, s);
         else sort_segments<kSortIPT>(c, pos, species, rec, n, s);
         const unsigned nbx = (nb + kXcds - 1) / kXcds * kXcds;
-        k_gather_parts<true><<<dim3(nbx), dim3(kBlock), 0, s>>>(rec, idx, c.parts, c.keys0, c.vals0, n, ts, lt);
+        k_gather_parts<true><<<dim3(nbx), dim3(kBlock), 0, s>>>(rec, idx, c.parts, c.keys0, c.vals0, n, ts, lt, cells);
     }
     return hipGetLastError();
 }

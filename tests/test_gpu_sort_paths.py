@@ -48,3 +48,23 @@ def test_stable_order(jtp, orc, kind, n):
             for dx in (0, 1):
                 occupied[(c[:, 2] + dz) % 64, (c[:, 1] + dy) % 64, (c[:, 0] + dx) % 64] = True
     assert np.all(rho.reshape(64, 64, 64)[~occupied] == 0)
+
+
+@pytest.mark.parametrize("precision,pm", [(0, 1), (0, 0), (1, 1)])
+@pytest.mark.parametrize("kind,n", [("random", 1), ("random", 2), ("equal", 2049), ("one segment", 2048), ("halo", 2047),
+                                    ("random", 128 * 2048), ("few", 128 * 2048 + 1), ("halo", 128 * 2048 + 255)])
+def test_group_cells(jtp, orc, kind, n, precision, pm):
+    """The gather's level-4 cell starts: the walk's groups are the runs of <= 32 in each cell, and cover every particle."""
+    print(f"case: group cells {kind} n={n} precision={precision} pm={pm}", flush=True)
+    rng = np.random.default_rng(n + 1)
+    pos = _positions(kind, n, rng)
+    sp = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int8)
+    p = jtp.default_params(250.0, 64)
+    p.precision, p.pm_enabled = precision, pm
+    ctx = jtp.ForceContext(p, 1.0, 1.0)
+    acc = jtp.DeviceArray.from_host(np.full((n, 3), np.nan, np.float64 if precision else np.float32))
+    dp, ds = jtp.DeviceArray.from_host(pos), jtp.DeviceArray.from_host(sp)
+    ctx.compute_forces_device(n, dp.ptr, ds.ptr, acc.ptr)
+    count = np.bincount((orc.morton(pos) >> np.uint64(51)).astype(np.int64), minlength=4096)
+    assert ctx.stats()["n_groups"] == np.sum((count + 31) // 32)
+    assert np.all(np.isfinite(acc.download()))
