@@ -449,16 +449,14 @@ int jtp_create(const jtp_params* p, jtp_ctx** out) {
     while (c.start_level < kGroupLevelBits && p->box_size / (double)(1 << (c.start_level + 1)) >= p->r_cut)
         ++c.start_level;
     if (e == hipSuccess) e = dalloc(c.dev_counters, kCtrTotal);
-    if (e == hipSuccess) e = dalloc(c.dev_inter, 2);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&c.host_pinned, 4 * sizeof(unsigned long long), 0);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c.host_status, kCtrStatus * sizeof(int32_t), 0);
     if (e == hipSuccess) e = dalloc(c.dev_step, 1);
     if (e == hipSuccess) e = dalloc(c.diag_scratch, kDiagScratch);
     if (e == hipSuccess) e = hipHostMalloc((void**)&c.host_step, sizeof(StepParams), 0);
     make_split_poly(c);
     if (e == hipSuccess) e = pm_tables(c);
     if (e == hipSuccess) {
-        for (int i = 0; i < 10 && e == hipSuccess; ++i) e = hipEventCreate(&c.ev[i]);
-        for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreate(&c.ev_build[i]);
+        for (int i = 0; i < Ctx::kEvents && e == hipSuccess; ++i) e = hipEventCreate(&c.ev[i]);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&c.fork_ev, hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&c.join_ev, hipEventDisableTiming);
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking);  // default priority
@@ -483,16 +481,14 @@ int jtp_destroy(jtp_ctx* h) {
     if (c.graph.capture_stream) (void)hipStreamDestroy(c.graph.capture_stream);
     void* ptrs[] = {c.rho, c.phi, c.rho2, c.phi2, c.grad, c.grad2, c.spec, c.spec2, c.twiddle, c.gtab, c.cell_start,
                     c.tile_start, c.dep_tbuf,
-                    c.cell4, c.cellnode, c.dev_counters, c.dev_inter, c.dense_slot, c.dev_step, c.diag_scratch,
+                    c.cell4, c.cellnode, c.dev_counters, c.dense_slot, c.dev_step, c.diag_scratch,
                     c.pot_short, c.acc_scratch, c.kself, c.seg, c.dev_fit64};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
-    if (c.host_pinned) (void)hipHostFree(c.host_pinned);
+    if (c.host_status) (void)hipHostFree(c.host_status);
     if (c.host_step) (void)hipHostFree(c.host_step);
-    for (int i = 0; i < 10; ++i)
+    for (int i = 0; i < Ctx::kEvents; ++i)
         if (c.ev[i]) (void)hipEventDestroy(c.ev[i]);
-    for (int i = 0; i < 2; ++i)
-        if (c.ev_build[i]) (void)hipEventDestroy(c.ev_build[i]);
     if (c.fork_ev) (void)hipEventDestroy(c.fork_ev);
     if (c.join_ev) (void)hipEventDestroy(c.join_ev);
     if (c.side) (void)hipStreamDestroy(c.side);
@@ -525,39 +521,35 @@ static int enqueue_prep(Ctx& c, int64_t n, const uint32_t* d_pos, const int8_t* 
                                c.p.tree_enabled ? c.cell4 : nullptr, s));
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[1], s));
     // The tree build and the PM phases only share read-only inputs (sorted keys and records), so the
-    // build runs on the side stream while the PM phases run on `s`; the walk waits for both.
-    const bool fork = c.p.tree_enabled && c.p.pm_enabled;
+    // build runs on the side stream while the PM phases run on `s`; the walk waits for both.  A timed evaluation
+    // forks and joins on the events of its phases: each record is a packet that its stream waits for (419 -> 403 us
+    // a force at 2e4 particles with seven of them instead of twelve and one status copy instead of four).
+    const bool tree = c.p.tree_enabled, pm = c.p.pm_enabled, fork = tree && pm;
+    const hipEvent_t forked = timed ? c.ev[1] : c.fork_ev, built = timed ? c.ev[2] : c.join_ev;
+    hipStream_t bs = fork ? c.side : s;
     if (fork) {
-        JTP_HIP(&c, hipEventRecord(c.fork_ev, s));
-        JTP_HIP(&c, hipStreamWaitEvent(c.side, c.fork_ev, 0));
-        if (timed) JTP_HIP(&c, hipEventRecord(c.ev_build[0], c.side));
-        JTP_HIP(&c, build_tree(c, n, c.side));
-        if (timed) JTP_HIP(&c, hipEventRecord(c.ev_build[1], c.side));
-        JTP_HIP(&c, hipEventRecord(c.join_ev, c.side));
-    } else if (c.p.tree_enabled) {
-        if (timed) JTP_HIP(&c, hipEventRecord(c.ev_build[0], s));
-        JTP_HIP(&c, build_tree(c, n, s));
-        if (timed) JTP_HIP(&c, hipEventRecord(c.ev_build[1], s));
+        if (!timed) JTP_HIP(&c, hipEventRecord(forked, s));
+        JTP_HIP(&c, hipStreamWaitEvent(bs, forked, 0));
     }
-    if (timed) JTP_HIP(&c, hipEventRecord(c.ev[2], s));
-    if (c.p.pm_enabled) JTP_HIP(&c, pm_deposit(c, n, s));
-    if (timed) JTP_HIP(&c, hipEventRecord(c.ev[3], s));
-    if (c.p.pm_enabled) JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, c.rho2, c.phi2, s));  // rho2: null without interlacing
-    if (timed) JTP_HIP(&c, hipEventRecord(c.ev[4], s));
-    if (c.p.pm_enabled) JTP_HIP(&c, pm_interp(c, n, s));
-    if (timed) JTP_HIP(&c, hipEventRecord(c.ev[5], s));
-    if (fork) JTP_HIP(&c, hipStreamWaitEvent(s, c.join_ev, 0));
+    if (tree) {
+        JTP_HIP(&c, build_tree(c, n, bs));
+        if (fork || timed) JTP_HIP(&c, hipEventRecord(built, bs));
+    }
+    if (pm) {
+        JTP_HIP(&c, pm_deposit(c, n, s));
+        if (timed) JTP_HIP(&c, hipEventRecord(c.ev[3], s));
+        JTP_HIP(&c, pm_fft_solve(c, c.rho, c.phi, c.rho2, c.phi2, s));  // rho2: null without interlacing
+        if (timed) JTP_HIP(&c, hipEventRecord(c.ev[4], s));
+        JTP_HIP(&c, pm_interp(c, n, s));
+        if (timed) JTP_HIP(&c, hipEventRecord(c.ev[5], s));
+    }
+    if (fork) JTP_HIP(&c, hipStreamWaitEvent(s, built, 0));
     return JTP_OK;
 }
 
-// Status words of an evaluation: interaction counts, group count, walk error flag, root flag.
-static int enqueue_status(Ctx& c, int64_t n, hipStream_t s) {
-    JTP_HIP(&c, hipMemcpyAsync(c.host_pinned, c.dev_inter, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    JTP_HIP(&c, hipMemcpyAsync(c.host_pinned + 3, c.dev_inter + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    JTP_HIP(&c, hipMemcpyAsync(c.host_pinned + 1, c.dev_counters, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    if (c.p.tree_enabled && n >= 2)
-        JTP_HIP(&c, hipMemcpyAsync((int32_t*)(c.host_pinned + 2), c.dev_counters + kCtrRoot, sizeof(int32_t),
-                                   hipMemcpyDeviceToHost, s));
+// Status words of an evaluation: group count, walk error flag, root flag, interaction counts.
+static int enqueue_status(Ctx& c, hipStream_t s) {
+    JTP_HIP(&c, hipMemcpyAsync(c.host_status, c.dev_counters, kCtrStatus * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     return JTP_OK;
 }
 
@@ -565,22 +557,21 @@ static int enqueue_forces(Ctx& c, int64_t n, const uint32_t* d_pos, const int8_t
                           hipStream_t s, bool timed, double* pot = nullptr) {
     int rc = enqueue_prep(c, n, d_pos, d_species, s, timed);
     if (rc != JTP_OK) return rc;
-    if (timed) JTP_HIP(&c, hipEventRecord(c.ev[7], s));
     if (c.p.tree_enabled) JTP_HIP(&c, walk(c, n, d_acc, s, pot));
     else JTP_HIP(&c, write_pm_only(c, n, d_acc, s));
     if (timed) JTP_HIP(&c, hipEventRecord(c.ev[6], s));
-    return enqueue_status(c, n, s);
+    return enqueue_status(c, s);
 }
 
 // Interprets the status words of the last force evaluation (after the stream synchronised).
 static int check_status(Ctx& c, int64_t n) {
     c.have_result = true;
     if (c.p.tree_enabled) {
-        const int32_t* cnt = (const int32_t*)(c.host_pinned + 1);
-        if (n >= 2 && ((const int32_t*)(c.host_pinned + 2))[0] != 1)
+        const int32_t* cnt = c.host_status;
+        if (n >= 2 && cnt[kCtrRoot] != 1)
             return fail(&c, JTP_ERR_STATE, "bottom-up pass did not reach the root (malformed hierarchy)");
-        if (cnt[1] == 1) return fail(&c, JTP_ERR_OVERFLOW, "walk stack overflow: a group's traversal exceeded the stack bound");
-        if (cnt[1] != 0) return fail(&c, JTP_ERR_STATE, "walk found a malformed hierarchy (code " + std::to_string(cnt[1]) + ")");
+        if (cnt[kCtrErr] == 1) return fail(&c, JTP_ERR_OVERFLOW, "walk stack overflow: a group's traversal exceeded the stack bound");
+        if (cnt[kCtrErr] != 0) return fail(&c, JTP_ERR_STATE, "walk found a malformed hierarchy (code " + std::to_string(cnt[kCtrErr]) + ")");
     }
     return JTP_OK;
 }
@@ -727,7 +718,7 @@ int jtp_step(jtp_ctx* h, int64_t n, uint32_t* d_pos, void* d_vel, const int8_t* 
         rc = ensure_graph(c, n, d_pos, d_vel, d_species, d_acc, scheme, s);
         if (rc != JTP_OK) return rc;
     }
-    JTP_HIP(&c, hipEventRecord(c.ev[8], s));
+    JTP_HIP(&c, hipEventRecord(c.ev[7], s));
     JTP_HIP(&c, hipMemcpyAsync(c.dev_step, c.host_step, sizeof(StepParams), hipMemcpyHostToDevice, s));
     if (use_graph) {
         JTP_HIP(&c, hipGraphLaunch(c.graph.exec, s));
@@ -735,7 +726,7 @@ int jtp_step(jtp_ctx* h, int64_t n, uint32_t* d_pos, void* d_vel, const int8_t* 
         rc = enqueue_step(c, n, d_pos, d_vel, d_species, d_acc, scheme, s, true);
         if (rc != JTP_OK) return rc;
     }
-    JTP_HIP(&c, hipEventRecord(c.ev[9], s));
+    JTP_HIP(&c, hipEventRecord(c.ev[8], s));
     JTP_HIP(&c, hipStreamSynchronize(s));
     return check_status(c, n);
 }
@@ -951,14 +942,22 @@ int jtp_get_stats(jtp_ctx* h, jtp_stats* out) {
     // the total covers the force call, or the whole step with its kicks and drifts
     float ms[6] = {-1, -1, -1, -1, -1, -1};
     if (c.last_kind < 2) {
-        // sort ev0-ev1; build on its own events (side stream); deposit ev2-ev3, FFT ev3-ev4,
-        // interpolation ev4-ev5; walk ev7-ev6 (ev7 follows the wait for the build)
+        // sort ev0-ev1; build ev1-ev2 (side stream); deposit ev1-ev3, FFT ev3-ev4, interpolation ev4-ev5; walk from
+        // the later of ev2 and ev5 to ev6
+        const bool tree = c.p.tree_enabled, pm = c.p.pm_enabled;
         JTP_HIP(&c, hipEventSynchronize(c.ev[6]));
         JTP_HIP(&c, hipEventElapsedTime(&ms[0], c.ev[0], c.ev[1]));
-        if (c.p.tree_enabled) JTP_HIP(&c, hipEventElapsedTime(&ms[1], c.ev_build[0], c.ev_build[1]));
-        else ms[1] = 0;
-        for (int i = 2; i < 5; ++i) JTP_HIP(&c, hipEventElapsedTime(&ms[i], c.ev[i], c.ev[i + 1]));
-        JTP_HIP(&c, hipEventElapsedTime(&ms[5], c.ev[7], c.ev[6]));
+        JTP_HIP(&c, hipEventElapsedTime(&ms[5], c.ev[tree ? 2 : pm ? 5 : 1], c.ev[6]));
+        for (int i = 1; i < 5; ++i) ms[i] = 0;
+        if (tree) JTP_HIP(&c, hipEventElapsedTime(&ms[1], c.ev[1], c.ev[2]));
+        if (pm) {
+            float since = 0;
+            JTP_HIP(&c, hipEventElapsedTime(&ms[2], c.ev[1], c.ev[3]));
+            JTP_HIP(&c, hipEventElapsedTime(&ms[3], c.ev[3], c.ev[4]));
+            JTP_HIP(&c, hipEventElapsedTime(&ms[4], c.ev[4], c.ev[5]));
+            JTP_HIP(&c, hipEventElapsedTime(&since, c.ev[5], c.ev[6]));
+            ms[5] = std::min(ms[5], since);
+        }
     }
     out->ms_sort = ms[0];
     out->ms_build = ms[1];
@@ -970,13 +969,13 @@ int jtp_get_stats(jtp_ctx* h, jtp_stats* out) {
     if (c.last_kind == 0) {
         JTP_HIP(&c, hipEventElapsedTime(&tot, c.ev[0], c.ev[6]));
     } else if (c.last_kind != 3) {
-        JTP_HIP(&c, hipEventSynchronize(c.ev[9]));
-        JTP_HIP(&c, hipEventElapsedTime(&tot, c.ev[8], c.ev[9]));
+        JTP_HIP(&c, hipEventSynchronize(c.ev[8]));
+        JTP_HIP(&c, hipEventElapsedTime(&tot, c.ev[7], c.ev[8]));
     }
     out->ms_total = tot;
-    out->interactions = c.host_pinned[0];
-    out->interactions_mono = c.host_pinned[3];
-    out->n_groups = ((const int32_t*)(c.host_pinned + 1))[0];
+    out->interactions = c.status_inter(0);
+    out->interactions_mono = c.status_inter(1);
+    out->n_groups = c.host_status[kCtrNGroups];
     return JTP_OK;
 }
 
@@ -1305,7 +1304,7 @@ static int ens_enqueue(jtp_ensemble* e, const int64_t* n, const uint32_t* const*
         ctrl += (size_t)walk_ctrl_size(m);
     }
     for (int b : batched) {
-        int rc = enqueue_status(e->boxes[b]->c, n[b], s);
+        int rc = enqueue_status(e->boxes[b]->c, s);
         if (rc != JTP_OK) return ens_fail(e, rc, "box " + std::to_string(b) + ": " + e->boxes[b]->c.err);
     }
     return JTP_OK;
@@ -1412,9 +1411,9 @@ int jtp_ensemble_get_stats(jtp_ensemble* e, int32_t box, jtp_stats* out) {
     for (jtp_ctx* h : e->boxes) {
         const Ctx& c = h->c;
         if (c.last_n <= 0) continue;
-        out->interactions += c.host_pinned[0];
-        out->interactions_mono += c.host_pinned[3];
-        out->n_groups += ((const int32_t*)(c.host_pinned + 1))[0];
+        out->interactions += c.status_inter(0);
+        out->interactions_mono += c.status_inter(1);
+        out->n_groups += c.host_status[kCtrNGroups];
         out->n_particles += c.last_n;
     }
     return JTP_OK;

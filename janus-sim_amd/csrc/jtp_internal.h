@@ -34,6 +34,8 @@ constexpr int kXcds = 8;             // MI355X accelerator complex dies; workgro
 // device counter block (int32): offsets
 constexpr int kCtrNGroups = 0, kCtrErr = 1, kCtrEarly = 2, kCtrDense = 3, kCtrInterp = 4;  // kCtrInterp: 3 words
 constexpr int kCtrRoot = 7;                         // 1: the build completed the root
+constexpr int kCtrInter = 32;                       // two 64-bit interaction counts, in a line of their own
+constexpr int kCtrStatus = kCtrInter + 4;           // words that the host reads after an evaluation, in one copy
 constexpr int kCtrXcd = 64;                         // kXcds walk-queue heads, kCtrXcdStride apart
 constexpr int kCtrXcdStride = 64;                   // 256 bytes: their atomics do not share a line
 constexpr int kCtrTotal = kCtrXcd + kXcds * kCtrXcdStride;
@@ -176,7 +178,6 @@ struct Ctx {
     int32_t *cellnode = nullptr;     // node holding each Morton cell of level start_level (<= 4096)
     int start_level = 4;             // finest level whose cell edge L / 2^level is >= r_cut (2..4)
     int32_t *dev_counters = nullptr; // kCtr* layout
-    unsigned long long *dev_inter = nullptr;  // interaction counter
     // PM
     int32_t *cell_start = nullptr;   // FP64: G^3 + 1 first sorted particle of each cell
     int32_t *tile_start = nullptr;   // FP32: G^3 / 512 + 1 first sorted particle of each 8^3-cell tile
@@ -200,7 +201,9 @@ struct Ctx {
     float poly_tscale_m = 0.0f;  // monopoles
     float poly_rho2_tail = 0.0f; // erfc + Gaussian monopoles: rho^2 beyond which the force is dropped
     double green_norm = 0.0;
-    unsigned long long* host_pinned = nullptr;  // [0] interactions, [1] (n_groups | err << 32)
+    int32_t* host_status = nullptr;  // the first kCtrStatus counters after an evaluation (pinned)
+    unsigned long long* dev_inter() const { return (unsigned long long*)(dev_counters + kCtrInter); }
+    unsigned long long status_inter(int k) const { return ((const unsigned long long*)(host_status + kCtrInter))[k]; }
 
     double* diag_scratch = nullptr;   // FP64 reduction partials (kDiagBlocks x 8) + 10 results
     double* pot_short = nullptr;      // energy diagnostic: short-range potential per particle (cap_n)
@@ -218,10 +221,10 @@ struct Ctx {
     int64_t last_n = -1;
     bool have_result = false;
     int last_kind = 0;                // 0 force call, 1 eager step, 2 graph step, 3 ensemble graph
-    // ev[0..6]: force phase boundaries, ev[7]: walk start; ev[8], ev[9]: step begin / end;
-    // ev_build[2]: the tree build on the side stream
-    hipEvent_t ev[10]{};
-    hipEvent_t ev_build[2]{};
+    // ev[0]: force begin; ends of the sort [1], the build (side stream) [2], the deposit [3], the FFT [4], the
+    // interpolation [5], the walk [6]; step begin [7] and end [8]
+    static constexpr int kEvents = 9;
+    hipEvent_t ev[kEvents]{};
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     hipStream_t side = nullptr;       // the tree build runs here, concurrently with the PM phases
     bool events_ok = false;

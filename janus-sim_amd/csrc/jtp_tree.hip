@@ -596,16 +596,15 @@ __global__ void k_groups(const uint64_t* __restrict__ keys, int64_t n, const int
 // Clears what an evaluation counts, the cells' starts (cell4), and the start cells of the walk: cellnode[c] is the node whose leaves are exactly
 // the particles of Morton cell c of level start_level (such a prefix range is one subtree; ~leaf for a single particle,
 // kNoNode for none), written by the build; the walk seeds each group's traversal with the 27 cells around it.
-__global__ void k_reset(int32_t* __restrict__ counters, int32_t* __restrict__ inter, int32_t* __restrict__ cellnode,
+__global__ void k_reset(int32_t* __restrict__ counters, int32_t* __restrict__ cellnode,
                         int32_t* __restrict__ cell4) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < 4096) cellnode[i] = kNoNode;
     if (i < kNCell4) cell4[i] = kNoCell;
     if (i < kCtrTotal) counters[i] = 0;
-    if (i < 4) inter[i] = 0;
 }
 hipError_t launch_reset(Ctx& c, hipStream_t s) {
-    k_reset<<<dim3(16), dim3(256), 0, s>>>(c.dev_counters, (int32_t*)c.dev_inter, c.cellnode, c.cell4);
+    k_reset<<<dim3(16), dim3(256), 0, s>>>(c.dev_counters, c.cellnode, c.cell4);
     return hipGetLastError();
 }
 

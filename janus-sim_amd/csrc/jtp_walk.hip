@@ -772,7 +772,7 @@ static void fill_args(Ctx& c, int64_t n, void* acc_out, WalkArgs& a) {
     a.early = c.early;
     a.early_max = (int32_t)early_cap(c.cap_n);
     a.counters = c.dev_counters;
-    a.inter = c.dev_inter;
+    a.inter = c.dev_inter();
     a.pm_acc = c.p.pm_enabled ? c.pm_acc : nullptr;
     a.perm = c.vals0;
     a.out = acc_out;
