@@ -839,10 +839,17 @@ __device__ inline void dft_small(const Cplx<R>* v, Cplx<R>* y, bool inv) {
     }
 }
 
+template <bool WAVE>
+__device__ inline void fft_barrier() {
+    if constexpr (WAVE) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    else __syncthreads();
+}
+
 // One Stockham stage of radix 2^LR after LS bits (Ns = 2^LS): butterfly j reads points
 // j + r G / RAD, multiplies point r by W_{RAD Ns}^{r k} (k = j mod Ns, tw[m] = e^{-2 pi i m / G}),
 // and writes output r to ((j / Ns) RAD Ns + k) + r Ns; all reads, a barrier, all writes.
-template <typename R, int LG, int LP, FftMap MAP, int LR, int LS, int T>
+// WAVE: T threads of one wavefront, ordered among themselves only.
+template <typename R, int LG, int LP, FftMap MAP, int LR, int LS, int T, bool WAVE>
 __device__ inline void fft_stage(Cplx<R>* buf, const Cplx<R>* tw, bool inv) {
 #pragma clang fp contract(off)
     constexpr int RAD = 1 << LR, G = 1 << LG, LNL = LP - LG, Q = G / RAD, LQ = LG - LR, Ns = 1 << LS;
@@ -873,34 +880,34 @@ __device__ inline void fft_stage(Cplx<R>* buf, const Cplx<R>* tw, bool inv) {
         ll[u] = l;
         oo[u] = ((j >> LS) << (LS + LR)) + k;
     }
-    __syncthreads();
+    fft_barrier<WAVE>();
 #pragma unroll
     for (int u = 0; u < NB; ++u)
 #pragma unroll
         for (int r = 0; r < RAD; ++r) buf[fft_at<LG, LP, MAP>(ll[u], oo[u] + r * Ns)] = y[u][r];
-    __syncthreads();
+    fft_barrier<WAVE>();
 }
 
 // Radix-8 stages while three or more bits remain, then one radix-4 or radix-2 stage
 // (G = 512: 8 8 8; 256: 8 8 4; 128: 8 8 2; 64: 8 8; 32: 8 4; 16: 8 2).
-template <typename R, int LG, int LP, FftMap MAP, int LS, int T>
+template <typename R, int LG, int LP, FftMap MAP, int LS, int T, bool WAVE>
 __device__ inline void fft_stages(Cplx<R>* buf, const Cplx<R>* tw, bool inv) {
     if constexpr (LG - LS >= 3) {
-        fft_stage<R, LG, LP, MAP, 3, LS, T>(buf, tw, inv);
-        fft_stages<R, LG, LP, MAP, LS + 3, T>(buf, tw, inv);
+        fft_stage<R, LG, LP, MAP, 3, LS, T, WAVE>(buf, tw, inv);
+        fft_stages<R, LG, LP, MAP, LS + 3, T, WAVE>(buf, tw, inv);
     } else if constexpr (LG - LS == 2) {
-        fft_stage<R, LG, LP, MAP, 2, LS, T>(buf, tw, inv);
+        fft_stage<R, LG, LP, MAP, 2, LS, T, WAVE>(buf, tw, inv);
     } else if constexpr (LG - LS == 1) {
-        fft_stage<R, LG, LP, MAP, 1, LS, T>(buf, tw, inv);
+        fft_stage<R, LG, LP, MAP, 1, LS, T, WAVE>(buf, tw, inv);
     }
 }
 
 // 2^LP / G lines of G points in LDS (fft_at), transformed in place by T threads; no FMA contraction, so every tile
 // size rounds each butterfly identically.
-template <typename R, int LG, int LP, FftMap MAP, int T = 256>
+template <typename R, int LG, int LP, FftMap MAP, int T = 256, bool WAVE = false>
 __device__ inline void lds_fft(Cplx<R>* buf, const Cplx<R>* __restrict__ tw, bool inv) {
     static_assert(LP >= LG && (1 << LP) / 8 >= T, "one radix-8 butterfly per thread and one line per block");
-    fft_stages<R, LG, LP, MAP, 0, T>(buf, tw, inv);
+    fft_stages<R, LG, LP, MAP, 0, T, WAVE>(buf, tw, inv);
 }
 
 // The meshes of one launch, or their half spectra: blockIdx.y = 0 or 1 (the two interlaced ones).
@@ -1140,8 +1147,10 @@ __global__ __launch_bounds__(256) void k_fft_z_inv(MeshPair<Cplx<R>> pair, const
 //
 // A plane of G x G reals is G / 2 packed complex lines.  After the x transforms the half spectra A, B of the two rows
 // of a line are unpacked in place, pair by pair: slots k and G - k hold Z[k] and Z[G - k] before, A[k] and B[k] after
-// (kPlane); slots 0 and G / 2 then hold (A[0], A[G/2]) and (B[0], B[G/2]), all real, so column 0 carries the columns 0 and
-// G / 2 as one complex sequence that is taken apart after the y transform.  T threads, a radix-8 butterfly each.
+// (kPlane); slots 0 and G / 2 then hold A[0] and B[0], and the real A[G/2] and B[G/2] are column G / 2, a line of its own
+// that a few threads of the first wavefront transform.  (Carried as the imaginary part of column 0 it costs nothing, but
+// rounds differently: with every column by itself each value is the one that the passes along x and y give, bit for bit,
+// and a trajectory does not depend on the path.)  T threads, a radix-8 butterfly each.
 //
 // Three launches a solve instead of five, and the half spectrum moved 4 times instead of 8; such meshes are bound by the
 // launches and each workgroup's chain of LDS stages (one mesh of 128 planes fills half the CUs).  Measured, with both
@@ -1156,6 +1165,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R
     constexpr int G = 1 << LG, H = G / 2 + 1, LP = 2 * LG - 1, T = plane_threads<LG>();
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[G];
+    __shared__ Cplx<R> half[G];  // column G / 2
     const int tid = threadIdx.x;
     for (int i = tid; i < G; i += T) stw[i] = tw[i];
     const R* __restrict__ src = real.mine() + (int64_t)blockIdx.x * G * G;
@@ -1181,25 +1191,22 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_xy(MeshPair<const R
         Cplx<R>& w = buf[fft_slot((p << LG) + (k == 0 ? G / 2 : G - k))];
         const Cplx<R> z = u, zc = w;
         if (k == 0) {
-            u = {z.x, zc.x};
-            w = {z.y, zc.y};
+            u = {z.x, (R)0};
+            w = {z.y, (R)0};
+            half[fft_slot(2 * p)] = {zc.x, (R)0};
+            half[fft_slot(2 * p + 1)] = {zc.y, (R)0};
         } else {
             u = {(R)0.5 * (z.x + zc.x), (R)0.5 * (z.y - zc.y)};  // A = (Z[k] + conj Z[G-k]) / 2
             w = {(R)0.5 * (z.y + zc.y), (R)0.5 * (zc.x - z.x)};  // B = (Z[k] - conj Z[G-k]) / (2i)
         }
     }
     __syncthreads();
+    if (tid < G / 8) lds_fft<R, LG, LG, kLines, G / 8, true>(half, stw, false);
     lds_fft<R, LG, LP, kPlane, T>(buf, stw, false);
     Cplx<R>* __restrict__ dst = spec.mine() + (int64_t)blockIdx.x * G * H;
     for (int e = tid; e < G * H; e += T) {
         const int r = e / H, k = e - r * H;
-        Cplx<R> o = buf[fft_at<LG, LP, kPlane>(k & (G / 2 - 1), r)];
-        if ((k & (G / 2 - 1)) == 0) {
-            const Cplx<R> n = buf[fft_at<LG, LP, kPlane>(0, (G - r) & (G - 1))];
-            o = k == 0 ? Cplx<R>{(R)0.5 * (o.x + n.x), (R)0.5 * (o.y - n.y)}
-                       : Cplx<R>{(R)0.5 * (o.y + n.y), (R)0.5 * (n.x - o.x)};
-        }
-        dst[e] = o;
+        dst[e] = k == G / 2 ? half[fft_slot(r)] : buf[fft_at<LG, LP, kPlane>(k, r)];
     }
 }
 
@@ -1210,24 +1217,18 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(MeshPair<Cplx<R>
     constexpr int G = 1 << LG, H = G / 2 + 1, LP = 2 * LG - 1, T = plane_threads<LG>();
     __shared__ Cplx<R> buf[1 << LP];
     __shared__ Cplx<R> stw[G];
+    __shared__ Cplx<R> half[G];  // column G / 2
     const int tid = threadIdx.x;
     for (int i = tid; i < G; i += T) stw[i] = tw[i];
     const Cplx<R>* __restrict__ src = spec.mine() + (int64_t)blockIdx.x * G * H;
 #pragma unroll 4
     for (int e = tid; e < G * G / 2; e += T) {
         const int r = e >> (LG - 1), k = e & (G / 2 - 1);
-        Cplx<R> v = src[r * H + k];
-        if (k == 0) {
-            // columns 0 and G / 2 become real in the y transform: their Hermitian parts, packed
-            const int n = (G - r) & (G - 1);
-            const Cplx<R> w = src[n * H], x = src[r * H + G / 2], y = src[n * H + G / 2];
-            const Cplx<R> f = {(R)0.5 * (v.x + w.x), (R)0.5 * (v.y - w.y)};
-            const Cplx<R> g = {(R)0.5 * (x.x + y.x), (R)0.5 * (x.y - y.y)};
-            v = {f.x - g.y, f.y + g.x};
-        }
-        buf[fft_at<LG, LP, kPlane>(k, r)] = v;
+        buf[fft_at<LG, LP, kPlane>(k, r)] = src[r * H + k];
     }
+    for (int r = tid; r < G; r += T) half[fft_slot(r)] = src[r * H + G / 2];
     __syncthreads();
+    if (tid < G / 8) lds_fft<R, LG, LG, kLines, G / 8, true>(half, stw, true);
     lds_fft<R, LG, LP, kPlane, T>(buf, stw, true);
 #pragma unroll 4
     for (int e = tid; e < G * G / 4; e += T) {
@@ -1237,7 +1238,7 @@ __global__ __launch_bounds__(plane_threads<LG>()) void k_fft_yx(MeshPair<Cplx<R>
         const Cplx<R> a = u, b = w;
         if (k == 0) {
             u = {a.x, b.x};
-            w = {a.y, b.y};
+            w = {half[fft_slot(2 * p)].x, half[fft_slot(2 * p + 1)].x};
         } else {
             u = {a.x - b.y, a.y + b.x};   // A + i B
             w = {a.x + b.y, -a.y + b.x};  // conj A + i conj B
