@@ -83,7 +83,7 @@ typedef struct jtp_params {
 typedef struct jtp_stats {
     double  ms_total;     /* force call, or the whole step (kicks, drifts) after jtp_step */
     double  ms_sort;      /* Morton keys + radix sort + particle gather        */
-    double  ms_build;     /* Karras hierarchy + bottom-up monopoles + groups   */
+    double  ms_build;     /* tree, monopoles and groups, from the end of the sort */
     double  ms_deposit;   /* deterministic CIC deposit (FP32: tile lists, per-tile
                              integer sums, face merge; FP64: cell offsets, gather) */
     double  ms_fft;       /* R2C, Green, C2R                                   */

@@ -1155,7 +1155,7 @@ __global__ __launch_bounds__(256) void k_fft_z_inv(MeshPair<Cplx<R>> pair, const
 // Three launches a solve instead of five, and the half spectrum moved 4 times instead of 8; such meshes are bound by the
 // launches and each workgroup's chain of LDS stages (one mesh of 128 planes fills half the CUs).  Measured, with both
 // interlaced meshes in the same launches, ms: 0.056 -> 0.025 at G = 32, 0.08 -> 0.033 at 64, 0.126 -> 0.070 at 128 (FP32);
-// one FP64 mesh at 128 with its call 0.077 -> 0.072.
+// one FP64 mesh at 128 with its call 0.077 -> 0.067.
 template <int LG> constexpr int plane_threads() { return LG == 7 ? 1024 : (LG == 6 ? 256 : 64); }
 
 template <typename R, int LG>
