@@ -111,22 +111,16 @@ static double split_excess_x3(double x) {
     return (split_direct(x, true) - 1.0) / (x * x * x);
 }
 
-// The same factors in extended precision for the FP64 walk's fits.  split_excess: (S - 1) / x^3 (erfc +
-// Gaussian) or (S - 1) / x (erfc only), by its series below x = 1/2, where the direct form cancels.
-static long double split_direct_l(long double x, bool gauss) {
-    return erfcl(x) + (gauss ? 2.0L * x / sqrtl((long double)M_PIl) * expl(-x * x) : 0.0L);
-}
-static long double split_excess_l(long double x, bool gauss) {
-    if (x >= 0.5L) return (split_direct_l(x, gauss) - 1.0L) / (gauss ? x * x * x : x);
-    // erf(x) = 2/sqrt(pi) sum (-1)^n x^{2n+1} / (n! (2n+1)); with the Gaussian term, see split_excess_x3
-    const long double x2 = x * x;
-    long double term = 1.0L, sum = 0.0L;  // gauss: x^{2n-2} / n! from n = 1; erfc only: x^{2n} / n! from n = 0
-    for (int n = gauss ? 1 : 0; n < 40; ++n) {
-        if (n > (gauss ? 1 : 0)) term *= x2 / n;
-        const long double w = gauss ? 2.0L * n / (2.0L * n + 1.0L) : -1.0L / (2.0L * n + 1.0L);
-        sum += (n & 1) ? -term * w : term * w;
+// erfcx(x) = exp(x^2) erfc(x) in extended precision for the FP64 walk's tables; beyond x = 10 by its asymptotic series
+// (the term left out there is below 1e-20).
+static long double erfcx_l(long double x) {
+    if (x < 10.0L) return expl(x * x) * erfcl(x);
+    long double term = 1.0L, sum = 1.0L;
+    for (int n = 1; n <= 12; ++n) {
+        term *= -(2.0L * n - 1.0L) / (2.0L * x * x);
+        sum += term;
     }
-    return 2.0L / sqrtl((long double)M_PIl) * sum;
+    return sum / (x * sqrtl((long double)M_PIl));
 }
 
 // Degree-deg Chebyshev interpolant of f on [a, b] as monomial coefficients of t = 2 (v - a) / (b - a) - 1, in
@@ -150,62 +144,54 @@ static void cheb_fit_l(long double a, long double b, int deg, double* out, F f) 
     for (int d = 0; d < N; ++d) out[d] = (double)mono[d];
 }
 
-// The FP64 fits in units of 2 r_s (x^2 for v): they depend on the law alone, so they are made once per process (0.4
-// ms) and scaled per context.  cut[i] covers sources cut at x <= kFit64Cut[i]; ok[i]: it and the other two are
-// within kFit64Tol of the law, relative to the Newtonian pair force.
-constexpr int kFit64Cuts = 2;
-constexpr double kFit64Cut[kFit64Cuts] = {2.3, 2.7};
+// The FP64 polynomials in units of 2 r_s depend on nothing, so they are made once per process (0.4 ms).  ok: all are
+// within kFit64Tol of what they stand for, in double as the kernel evaluates them.
 struct UnitFit64 {
-    double cut[kFit64Cuts][kFit64Pair + 1], tail[kFit64Tail + 1], far[kFit64Far + 1];
-    bool ok[kFit64Cuts];
-    explicit UnitFit64(bool gauss) {
-        auto excess = [&](long double y) { return split_excess_l(sqrtl(y), gauss); };
-        auto whole = [&](long double y) { return split_direct_l(sqrtl(y), gauss) / (y * sqrtl(y)); };
-        const long double y1 = (long double)kFit64X1 * kFit64X1, y2 = (long double)kFit64X2 * kFit64X2;
-        auto err = [&](long double a, long double b, int deg, const double* cf, bool full) {
+    double cut[kFit64CutDeg + 1], tail[kFit64TailDeg + 1], far[kFit64FarDeg + 1], ex[kFit64ExpDeg + 1];
+    bool ok;
+    UnitFit64() {
+        auto fit = [&](long double a, long double b, int deg, double* cf, auto f) {
+            cheb_fit_l(a, b, deg, cf, f);
             long double worst = 0;
             for (int i = 0; i <= 200; ++i) {
                 const long double y = a + (b - a) * (i + 0.01L) / 200.02L, t = 2.0L * (y - a) / (b - a) - 1.0L;
-                long double p = cf[deg];
-                for (int d = deg - 1; d >= 0; --d) p = p * t + cf[d];
-                const long double w = full || gauss ? y * sqrtl(y) : sqrtl(y);  // to the Newtonian force
-                worst = std::max(worst, fabsl(p - (full ? whole(y) : excess(y))) * w);
+                double p = cf[deg];
+                for (int d = deg - 1; d >= 0; --d) p = std::fma(p, (double)t, cf[d]);
+                worst = std::max(worst, fabsl(p / f(y) - 1.0L));
             }
-            return worst;
+            return worst < kFit64Tol;
         };
-        cheb_fit_l(0.0L, y1, kFit64Tail, tail, excess);
-        cheb_fit_l(y1, y2, kFit64Far, far, whole);
-        const bool rest = err(0.0L, y1, kFit64Tail, tail, false) < kFit64Tol && err(y1, y2, kFit64Far, far, true) < kFit64Tol;
-        for (int i = 0; i < kFit64Cuts; ++i) {
-            const long double yp = (long double)kFit64Cut[i] * kFit64Cut[i];
-            cheb_fit_l(0.0L, yp, kFit64Pair, cut[i], excess);
-            ok[i] = rest && err(0.0L, yp, kFit64Pair, cut[i], false) < kFit64Tol;
-        }
+        const long double z1 = 1.0L / ((long double)kFit64Tail * kFit64Tail);
+        const long double ln2 = logl(2.0L);
+        ok = fit(0.0L, kFit64Cut, kFit64CutDeg, cut, erfcx_l);
+        ok = fit(0.0L, kFit64Tail, kFit64TailDeg, tail, erfcx_l) && ok;
+        ok = fit(0.0L, z1, kFit64FarDeg, far, [](long double z) { return erfcx_l(1.0L / sqrtl(z)) / sqrtl(z); }) && ok;
+        ok = fit(-0.5L, 0.5L, kFit64ExpDeg, ex, [=](long double f) { return f == 0 ? ln2 : expm1l(f * ln2) / f; }) && ok;
+        for (int d = 0; d <= kFit64ExpDeg; ++d) ex[d] = std::ldexp(ex[d], d);  // of f instead of 2 f
     }
 };
 
 static void make_split_poly64(Ctx& c) {
     SplitPoly64& q = c.poly64;
     q = SplitPoly64{};
-    const bool gauss = c.p.split_mode == JTP_SPLIT_ERFC_GAUSS;
-    static const UnitFit64 unit_gauss(true), unit_erfc(false);
-    const UnitFit64& u = gauss ? unit_gauss : unit_erfc;
-    const double ci = 0.5 / c.p.r_s, ci3 = ci * ci * ci;
-    const double xp = std::sqrt(c.p.r_cut * c.p.r_cut + c.p.softening * c.p.softening) * ci * (1.0 + 1e-12);
-    int k = 0;
-    while (k < kFit64Cuts && !(xp <= kFit64Cut[k])) ++k;
-    if (k == kFit64Cuts || !u.ok[k]) return;
-    for (int d = 0; d <= kFit64Pair; ++d) q.cp[d] = u.cut[k][d] * (gauss ? ci3 : ci);
-    for (int d = 0; d <= kFit64Tail; ++d) q.ct[d] = u.tail[d] * (gauss ? ci3 : ci);
-    for (int d = 0; d <= kFit64Far; ++d) q.cg[d] = u.far[d] * ci3;
-    const double c2 = ci * ci, y1 = kFit64X1 * kFit64X1, y2 = kFit64X2 * kFit64X2;
-    q.sp = 2.0 * c2 / (kFit64Cut[k] * kFit64Cut[k]);
-    q.st = 2.0 * c2 / y1;
-    q.sg = 2.0 * c2 / (y2 - y1);
-    q.og = 2.0 * y1 / (y2 - y1) + 1.0;
-    q.v1 = y1 / c2;
-    q.v2 = y2 / c2;
-    q.ok = std::isfinite(ci3) && ci3 > 1e-280 && std::isfinite(q.v2) ? 1 : 0;
+    static const UnitFit64 u;
+    const long double ci = 0.5L / c.p.r_s, k = -ci * ci / logl(2.0L);
+    const double xp = (double)(std::sqrt(c.p.r_cut * c.p.r_cut + c.p.softening * c.p.softening) * ci) * (1.0 + 1e-12);
+    if (!u.ok || !(xp <= kFit64Cut)) return;
+    std::copy(std::begin(u.cut), std::end(u.cut), q.cp);
+    std::copy(std::begin(u.tail), std::end(u.tail), q.ct);
+    std::copy(std::begin(u.far), std::end(u.far), q.cf);
+    std::copy(std::begin(u.ex), std::end(u.ex), q.ce);
+    q.sp = (double)(2.0L * ci / kFit64Cut);
+    q.st = (double)(2.0L * ci / kFit64Tail);
+    q.sf = (double)(2.0L * kFit64Tail * kFit64Tail / (ci * ci));
+    q.kh = (double)k;
+    q.kl = (double)(k - q.kh);
+    q.g = (double)(2.0L * ci / sqrtl((long double)M_PIl));
+    q.rs2 = (double)(1.0L / ci);
+    q.v1 = (double)(kFit64Tail * kFit64Tail / (ci * ci));
+    q.vmax = (double)(-1080.0L / k);
+    q.ok = q.kh < -1e-280 && std::isfinite(q.kh) && std::isfinite(q.vmax) ? 1 : 0;
 }
 
 void make_split_poly(Ctx& c) {

@@ -98,24 +98,30 @@ struct SplitPoly {
     float cm[kPolyDeg + 1];
 };
 
-// Polynomials of the FP64 walk's erfc laws, v = rho^2 = r^2 + eps^2, x = rho / (2 r_s).  S - 1 is x^3 (erfc +
-// Gaussian) or x (erfc only) times an entire function of x^2, so S / rho^3 = 1 / rho^3 + H(v) or
-// 1 / rho^3 + E(v) / rho^2 with H, E polynomials to double precision:
-//  * cp: sources cut at r_cut (x <= 2.3, or 2.7 for r_cut above 4.6 r_s);
-//  * ct on [0, v1], x(v1) = kFit64X1 (1.8 r_cut at the default r_cut = 4.5 r_s): monopoles of nodes that straddle r_cut;
-//  * cg: S / rho^3 itself on [v1, v2], x(v2) = kFit64X2, where S < 1e-16; zero beyond.
-// `ok`: every fit is within kFit64Tol of the law, relative to the Newtonian pair force (r_cut up to 5.4 r_s);
-// otherwise the walk calls erfc and exp.
-constexpr int kFit64Pair = 20, kFit64Tail = 30, kFit64Far = 25;
-constexpr double kFit64X1 = 4.0, kFit64X2 = 6.2;
+// Tables of the FP64 walk's erfc laws.  With v = rho^2 = r^2 + eps^2 and x = rho / (2 r_s), S = exp(-x^2) (erfcx(x) [+
+// 2 x / sqrt(pi)]): a product and a sum of positive terms, so that no digit is lost where S is small.
+//  * erfcx: polynomials of x on [0, kFit64Cut] (pairs cut at r_cut) and on [0, kFit64Tail] (monopoles of nodes that straddle
+//    it); beyond, x erfcx(x) as a polynomial of 1 / x^2;
+//  * exp(-x^2) = 2^n (1 + f Q(f)), n + f = -x^2 / ln 2, |f| <= 1/2 (Cody and Waite's reduction, with the product kept exact by
+//    an FMA).
+// Error relative to the pair's own force, against 128-bit arithmetic: at most 7e-16 at every x, rms 1.6e-16 (erfc and exp of
+// a rounded x: 3.0e-15 for x <= 2.25, 8.3e-15 for x <= 4, 2.4e-14 for x <= 6.2; rms 4e-16, 1.4e-15, 5.7e-15).  1 / rho^3 plus a
+// polynomial, at 44 instructions a cut pair instead of 71, loses digits as S falls: 2.7e-14 at 2.25, 3e-9 at 4.
+// `ok`: the pairs' range covers r_cut (up to 5.4 r_s) and the polynomials, evaluated in double, are within kFit64Tol of
+// erfcx; otherwise the walk calls erfc and exp.
+constexpr int kFit64CutDeg = 24, kFit64TailDeg = 29, kFit64FarDeg = 13, kFit64ExpDeg = 10;
+constexpr double kFit64Cut = 2.7, kFit64Tail = 4.0;
 constexpr double kFit64Tol = 1e-15;
 struct SplitPoly64 {
-    double cp[kFit64Pair + 1];
-    double ct[kFit64Tail + 1];
-    double cg[kFit64Far + 1];
-    double sp, st;        // t = v * s - 1 of cp and ct
-    double sg, og;        // t = v * sg - og of cg
-    double v1, v2;
+    double cp[kFit64CutDeg + 1];   // of t = rho * sp - 1
+    double ct[kFit64TailDeg + 1];  // of t = rho * st - 1
+    double cf[kFit64FarDeg + 1];   // of t = sf / v - 1, times rho (in units of 2 r_s)
+    double ce[kFit64ExpDeg + 1];   // Q
+    double sp, st, sf;
+    double kh, kl;    // -x^2 / ln 2 = v (kh + kl)
+    double g;         // 2 x / sqrt(pi) = g rho
+    double rs2;       // 2 r_s
+    double v1, vmax;  // v of x = kFit64Tail; v from which on S is below the smallest double
     int32_t ok;
 };
 

@@ -134,51 +134,73 @@ struct Pair<float, MODE, CUT> {
     }
 };
 
-// 1 / sqrt(x), x > 0: the hardware estimate y (relative error below 2^-20) and one third-order step with the
-// residual e = 1 - x y^2, y (1 + e/2 + 3 e^2/8): the next term is below 2^-60.
-__device__ inline double rsqrt_pos(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = __builtin_fma(-(x * y), y, 1.0);
-    return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+// 1 / v^{3/2}, v > 0, within half an ulp and 2^-58: the hardware's estimate of 1 / sqrt(v) (within 2^-20) cut to 17 bits, y,
+// so that y^2 and y^3 are exact, times the series of (1 - e)^{-3/2} in the residual e = 1 - v y^2 < 2^-14.
+__device__ inline double inv_cube(double v) {
+    const double y = __hiloint2double(__double2hiint(__builtin_amdgcn_rsq(v)) & ~15, 0);
+    const double w = y * y, e = __builtin_fma(-v, w, 1.0), y3 = w * y;
+    return __builtin_fma(y3 * e, __builtin_fma(e, __builtin_fma(e, 35.0 / 16, 15.0 / 8), 1.5), y3);
 }
 
-// FP64 erfc laws without erfc and exp: S / rho^3 = 1 / rho^3 + H(rho^2) (erfc + Gaussian) or 1 / rho^3 + E(rho^2) /
-// rho^2 (erfc only).  VALU-bound: 44 instructions a cut pair, 52 a tail monopole.  Measured against OCML's erfc and exp
-// in the same loops: walk 24.9 -> 14.7 ms at 2.75e6 clustered particles, 6.2 -> 3.7 ms at 2 x 64^3; accelerations agree
-// to 2.7e-16 (2-norm).  Shorter lists for a third wave per SIMD (320 and 256 entries) are 3 and 10 % slower.
+// FP64 erfc laws without erfc and exp: S / rho^3 = exp(-x^2) (erfcx(x) [+ 2 x / sqrt(pi)]) / rho^3 (SplitPoly64).
+// VALU-bound: 71 instructions a cut pair, 80 a tail monopole.  Measured against OCML's erfc and exp in the same loops: a
+// force 6.97 -> 4.66 ms at 2 x 64^3 particles, 34.1 -> 19.7 ms at 2.75e6 clustered ones (3.4 and 15 ms with 1 / rho^3 plus a
+// polynomial, 44 instructions, which loses the small forces' digits); accelerations agree to 3e-16 (2-norm).  Shorter lists for
+// a third wave per SIMD (320 and 256 entries) were 3 and 10 % slower with that loop.
 using ConstFit = const __attribute__((address_space(4))) SplitPoly64;
-__device__ inline ConstFit* const_fit(const SplitPoly64* p) { return (ConstFit*)(uintptr_t)p; }
-
-template <int MODE>
-__device__ inline double fit_law(double p, double inv) {
-    const double inv2 = inv * inv;
-    return MODE == JTP_SPLIT_ERFC_GAUSS ? __builtin_fma(inv2, inv, p) : inv2 * (inv + p);
+// The table's address with its origin hidden, so that the coefficients are read where they are used and not held across
+// the traversal.
+__device__ inline ConstFit* const_fit(const WalkArgs& a) {
+    const SplitPoly64* p = a.fit64;
+    asm volatile("" : "+s"(p));
+    return (ConstFit*)(uintptr_t)p;
+}
+// Coefficients in vector registers: with all of a law's in scalar ones beside the walk's own arguments those spill (136 lane
+// reads a pair).
+template <int N>
+__device__ inline void vector_copy(double (&to)[N], const __attribute__((address_space(4))) double* from) {
+#pragma unroll
+    for (int d = 0; d < N; ++d) {
+        to[d] = from[d];
+        asm volatile("" : "+v"(to[d]));
+    }
 }
 
-// Sources cut at r_cut, `count` list entries from `L` in steps of `step`: the sums of f d.  The coefficients are read
-// here, each time (the asm hides the pointer's origin), into scalar registers, and not held across the traversal.
+// exp(-x^2) p i3 with -x^2 / ln 2 = v (kh + kl).  The multiple n of ln 2 comes from the low bits of a sum with 1.5 x 2^52.
+__device__ inline double times_exp(double p, double i3, double v, double kh, double kl,
+                                   const double (&ce)[kFit64ExpDeg + 1]) {
+    const double m = __builtin_fma(v, kh, 0x1.8p52);
+    const double f = __builtin_fma(v, kl, __builtin_fma(v, kh, -(m - 0x1.8p52)));
+    double q = ce[kFit64ExpDeg];
+#pragma unroll
+    for (int d = kFit64ExpDeg - 1; d >= 0; --d) q = __builtin_fma(q, f, ce[d]);
+    return __builtin_amdgcn_ldexp(__builtin_fma(p, q * f, p) * i3, __double2loint(m));
+}
+
+// Sources cut at r_cut, `count` list entries from `L` in steps of `step`: the sums of f d.
 template <int MODE>
 __device__ inline void fit_cut(const double4* L, int count, int step, double tx, double ty, double tz,
                                const WalkArgs& a, double eps2, double rcut2, double& px, double& py, double& pz) {
-    const SplitPoly64* raw = a.fit64;
-    asm volatile("" : "+s"(raw));
-    ConstFit* c = const_fit(raw);
-    double cp[kFit64Pair + 1];
+    ConstFit* c = const_fit(a);
+    double cp[kFit64CutDeg + 1], ce[kFit64ExpDeg + 1];
 #pragma unroll
-    for (int d = 0; d <= kFit64Pair; ++d) cp[d] = c->cp[d];
-    const double sp = c->sp;
+    for (int d = 0; d <= kFit64CutDeg; ++d) cp[d] = c->cp[d];
+    vector_copy(ce, c->ce);
+    const double sp = c->sp, g = c->g, kh = c->kh, kl = c->kl;
 #pragma unroll 4
     for (int j = 0; j < count; ++j) {
         const double4 e = L[j * step];
         const double dx = e.x - tx, dy = e.y - ty, dz = e.z - tz;
         const double r2 = dx * dx + dy * dy + dz * dz;
         const double v = r2 + eps2;
-        const double t = __builtin_fma(v, sp, -1.0);
-        double p = cp[kFit64Pair];
+        const double i3 = inv_cube(v), rho = v * (v * i3);
+        const double t = __builtin_fma(rho, sp, -1.0);
+        double p = cp[kFit64CutDeg];
 #pragma unroll
-        for (int d = kFit64Pair - 1; d >= 0; --d) p = __builtin_fma(p, t, cp[d]);
-        double f = e.w * fit_law<MODE>(p, rsqrt_pos(v));
-        f = r2 < rcut2 ? f : 0.0;  // on the product: the polynomial may be anything beyond its range
+        for (int d = kFit64CutDeg - 1; d >= 0; --d) p = __builtin_fma(p, t, cp[d]);
+        if (MODE == JTP_SPLIT_ERFC_GAUSS) p = __builtin_fma(rho, g, p);
+        double f = e.w * times_exp(p, i3, v, kh, kl, ce);
+        f = r2 < rcut2 ? f : 0.0;  // on the product: the polynomials may be anything beyond their range
         px += f * dx;
         py += f * dy;
         pz += f * dz;
@@ -186,24 +208,18 @@ __device__ inline void fit_cut(const double4* L, int count, int step, double tx,
 }
 
 // The monopoles of nodes that straddle r_cut, `count` list entries from `L` in steps of `step`: the sums of f d.
-// Four entries at a time share each coefficient, kept in vector registers: 31 of them in scalar ones beside the
-// walk's own arguments spilled (136 lane reads a pair, 221 instructions instead of 52).
+// Four entries at a time share each coefficient.
 template <int MODE>
 __device__ inline void fit_tail(const double4* L, int count, int step, double tx, double ty, double tz,
                                 const WalkArgs& a, double eps2, double& px, double& py, double& pz) {
-    const SplitPoly64* raw = a.fit64;
-    asm volatile("" : "+s"(raw));  // read here, each time: not held across the traversal
-    ConstFit* c = const_fit(raw);
-    double ct[kFit64Tail + 1];
-#pragma unroll
-    for (int d = 0; d <= kFit64Tail; ++d) {
-        ct[d] = c->ct[d];
-        asm volatile("" : "+v"(ct[d]));
-    }
-    const double st = c->st, v1 = c->v1;
+    ConstFit* c = const_fit(a);
+    double ct[kFit64TailDeg + 1], ce[kFit64ExpDeg + 1];
+    vector_copy(ct, c->ct);
+    vector_copy(ce, c->ce);
+    const double st = c->st, g = c->g, kh = c->kh, kl = c->kl, v1 = c->v1, vend = c->vmax;
     constexpr int U = 4;
     for (int j = 0; j < count; j += U) {
-        double dx[U], dy[U], dz[U], q[U], v[U], t[U], s[U];
+        double dx[U], dy[U], dz[U], q[U], v[U], i3[U], t[U], p[U];
         double vmax = 0.0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -214,32 +230,30 @@ __device__ inline void fit_tail(const double4* L, int count, int step, double tx
             dz[u] = e.z - tz;
             q[u] = in ? e.w : 0.0;
             v[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u] + eps2;
-            t[u] = __builtin_fma(v[u], st, -1.0);
-            s[u] = ct[kFit64Tail];
+            i3[u] = inv_cube(v[u]);
+            t[u] = __builtin_fma(v[u] * (v[u] * i3[u]), st, -1.0);
+            p[u] = ct[kFit64TailDeg];
             vmax = fmax(vmax, v[u]);
         }
 #pragma unroll
-        for (int d = kFit64Tail - 1; d >= 0; --d)
+        for (int d = kFit64TailDeg - 1; d >= 0; --d)
 #pragma unroll
-            for (int u = 0; u < U; ++u) s[u] = __builtin_fma(s[u], t[u], ct[d]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) s[u] = fit_law<MODE>(s[u], rsqrt_pos(v[u]));
+            for (int u = 0; u < U; ++u) p[u] = __builtin_fma(p[u], t[u], ct[d]);
         if (__any(vmax > v1)) {  // beyond 1.8 r_cut: the widest groups of thin regions
-            const SplitPoly64* raw2 = a.fit64;
-            asm volatile("" : "+s"(raw2));
-            ConstFit* c2 = const_fit(raw2);
-            const double v2 = c2->v2;
+            ConstFit* c2 = const_fit(a);
+            const double sf = c2->sf, rs2 = c2->rs2;
             for (int u = 0; u < U; ++u) {
-                const double tg = __builtin_fma(v[u], c2->sg, -c2->og);
-                double g = c2->cg[kFit64Far];
+                const double inv = v[u] * i3[u], tf = __builtin_fma(inv * inv, sf, -1.0);
+                double r = c2->cf[kFit64FarDeg];
 #pragma unroll
-                for (int d = kFit64Far - 1; d >= 0; --d) g = __builtin_fma(g, tg, c2->cg[d]);
-                s[u] = v[u] > v1 ? (v[u] < v2 ? g : 0.0) : s[u];
+                for (int d = kFit64FarDeg - 1; d >= 0; --d) r = __builtin_fma(r, tf, c2->cf[d]);
+                p[u] = v[u] > v1 ? r * (inv * rs2) : p[u];
             }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const double f = q[u] * s[u];
+            if (MODE == JTP_SPLIT_ERFC_GAUSS) p[u] = __builtin_fma(v[u] * (v[u] * i3[u]), g, p[u]);
+            const double f = q[u] * times_exp(p[u], i3[u], fmin(v[u], vend), kh, kl, ce);
             px += f * dx[u];
             py += f * dy[u];
             pz += f * dz[u];
