@@ -327,17 +327,18 @@ struct SortArgs {
     uint32_t* hi_out;
     uint8_t* lo_out;
     uint32_t* val_out;
-    uint32_t* hist;           // counts [tile][256], then (segments) each tile's first output position per digit
+    uint32_t* hist;           // counts [tile][256], then (segments) those of the segment's tiles before
     const uint32_t* seg_tot;  // particles of each segment; nullptr: one segment
+    uint32_t* dig_tot;        // segments: counts [segment][256]
     int32_t nblk;             // tiles (one segment)
     int32_t shift;            // of the digit in hi_in
 };
 
-// Tile `b` of the segments' tiles: its particles [base, base + cnt); false beyond the last.  256 threads or more, all
-// of them; seg >= 0 asks for a segment instead: base its start, cnt its tiles, b its first tile.
+// Tile `b` of the segments' tiles: its particles [base, base + cnt), its segment and that one's start; false beyond the last.
+// 256 threads or more, all of them; seg >= 0 asks for a segment instead: base its start, cnt its tiles, b its first tile.
 template <int TILE>
-__device__ inline bool seg_find(const uint32_t* __restrict__ tot, int seg, int& b, int64_t& base, int& cnt,
-                                uint32_t* lds /* 8 */) {
+__device__ inline bool seg_find(const uint32_t* __restrict__ tot, int& seg, int& b, int64_t& base, int& cnt,
+                                uint32_t& seg_start, uint32_t* lds /* 10 */) {
     const int t = threadIdx.x;
     if (t == 4) lds[4] = 0;
     const uint32_t c = t < kSegs ? tot[t] : 0;
@@ -354,6 +355,8 @@ __device__ inline bool seg_find(const uint32_t* __restrict__ tot, int seg, int& 
     }
     if (t < kSegs && (seg >= 0 ? t == seg : (uint32_t)b >= ti - nt && (uint32_t)b < ti)) {
         lds[4] = 1;
+        lds[8] = (uint32_t)t;
+        lds[9] = ci - c;
         if (seg >= 0) {
             lds[5] = ci - c;
             lds[6] = nt;
@@ -369,6 +372,8 @@ __device__ inline bool seg_find(const uint32_t* __restrict__ tot, int seg, int& 
     base = lds[5];
     cnt = (int)lds[6];
     b = (int)lds[7];
+    seg = (int)lds[8];
+    seg_start = lds[9];
     return lds[4] != 0;
 }
 
@@ -401,13 +406,14 @@ __global__ __launch_bounds__(256) void k_sort_keys(const uint32_t* __restrict__ 
 template <int IPT, int LO, bool SEG>
 __global__ __launch_bounds__(256) void k_sort_hist(SortArgs a) {
     __shared__ uint32_t h[256];
-    __shared__ uint32_t lds[8];
+    __shared__ uint32_t lds[10];
     const int tid = threadIdx.x;
     constexpr int TILE = 256 * IPT;
-    int b = (int)blockIdx.x, cnt;
+    int b = (int)blockIdx.x, cnt, seg = -1;
+    uint32_t seg_start = 0;
     int64_t base = (int64_t)b * TILE;
     if (SEG) {
-        if (!seg_find<TILE>(a.seg_tot, -1, b, base, cnt, lds)) return;
+        if (!seg_find<TILE>(a.seg_tot, seg, b, base, cnt, seg_start, lds)) return;
     } else {
         cnt = a.n - base < TILE ? (int)(a.n - base) : TILE;
     }
@@ -426,37 +432,34 @@ __global__ __launch_bounds__(256) void k_sort_hist(SortArgs a) {
     a.hist[(int64_t)b * 256 + tid] = h[tid];
 }
 
-// One workgroup per segment: its tiles' counts -> the first output position of each (tile, digit).  Four groups of 256
-// threads (a thread per digit) take a quarter of the tiles each.
-template <int TILE>
+// Each tile's counts -> those of its segment's tiles before it, and the segment's counts.  A workgroup takes DIG digits of one
+// segment, its 1024 / DIG groups of threads a run of the tiles each.  Several workgroups a segment, because a set may lie in
+// one of them: with one each and four runs a digit, 4.1e6 particles of one octant cell took 1.50 ms to sort (1.22 with 32
+// digits a workgroup, 1.34 with 128) and 2.2e7 took 2.75 (2.41; 2.48 with 64).  The workgroups cost 3 us a pass at 32 digits
+// where the tiles are few, nothing at 128 (3e5 and 1e6 particles in a full box: 0.10 and 0.13 ms to sort; with 32 0.11 and 0.15).
+constexpr int64_t kScanWide = (int64_t)2 << 20;  // 32 digits from this many particles (4.1e6 crowded: 1.88 ms a call before
+                                                // the segments, 1.93 with 128 digits, 1.85 with 32)
+template <int TILE, int DIG>
 __global__ __launch_bounds__(1024) void k_sort_segscan(SortArgs a) {
-    __shared__ uint32_t part[4][256];
-    __shared__ uint32_t lds[8], wl[4];
-    const int g = threadIdx.x >> 8, d = threadIdx.x & 255;
-    int first = 0, nt;
+    constexpr int RUNS = 1024 / DIG;
+    __shared__ uint32_t part[RUNS][DIG];
+    __shared__ uint32_t lds[10];
+    const int g = threadIdx.x / DIG, dd = threadIdx.x % DIG, d = (int)blockIdx.y * DIG + dd;
+    int seg = (int)blockIdx.x, first = 0, nt;
+    uint32_t seg_start;
     int64_t start;
-    if (!seg_find<TILE>(a.seg_tot, (int)blockIdx.x, first, start, nt, lds)) return;
+    if (!seg_find<TILE>(a.seg_tot, seg, first, start, nt, seg_start, lds)) return;
     if (nt == 0) return;
-    const int q = (nt + 3) / 4, t0 = g * q < nt ? g * q : nt, t1 = t0 + q < nt ? t0 + q : nt;
+    const int q = (nt + RUNS - 1) / RUNS, t0 = g * q < nt ? g * q : nt, t1 = t0 + q < nt ? t0 + q : nt;
     uint32_t* h = a.hist + (int64_t)first * 256 + d;
     uint32_t s = 0;
 #pragma unroll 8
     for (int t = t0; t < t1; ++t) s += h[(int64_t)t * 256];
-    part[g][d] = s;
+    part[g][dd] = s;
     __syncthreads();
-    uint32_t before = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t v = part[i][d];
-        if (i < g) before += v;
-        tot += v;
-    }
-    // exclusive scan of the digits' totals (every group does it: 256 threads each)
-    const uint32_t incl = (uint32_t)wave_incl_scan_dpp((int)tot);
-    if (g == 0 && (d & 63) == 63) wl[d >> 6] = incl;
-    __syncthreads();
-    uint32_t run = (uint32_t)start + incl - tot + before;
-    for (int i = 0; i < (d >> 6); ++i) run += wl[i];
+    uint32_t run = 0;
+    for (int i = 0; i < g; ++i) run += part[i][dd];
+    if (g == RUNS - 1) a.dig_tot[seg * 256 + d] = run + s;
 #pragma unroll 8
     for (int t = t0; t < t1; ++t) {
         const uint32_t v = h[(int64_t)t * 256];
@@ -513,15 +516,16 @@ __global__ __launch_bounds__(256) void k_sort_scatter(SortArgs a) {
     using LoT = typename std::conditional<LO == 16, uint16_t, uint8_t>::type;
     __shared__ uint16_t wcnt[4][256];
     __shared__ uint32_t gbase[256];
-    __shared__ uint32_t lds[8];
+    __shared__ uint32_t lds[10];
     __shared__ uint32_t shi[TILE];
     __shared__ uint32_t sval[TILE];
     __shared__ LoT slo[LO ? TILE : 1];
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    int b = (int)blockIdx.x, cnt;
+    int b = (int)blockIdx.x, cnt, seg = -1;
+    uint32_t seg_start = 0;
     int64_t base = (int64_t)b * TILE;
     if (SEG) {
-        if (!seg_find<TILE>(a.seg_tot, -1, b, base, cnt, lds)) return;
+        if (!seg_find<TILE>(a.seg_tot, seg, b, base, cnt, seg_start, lds)) return;
     } else {
         cnt = a.n - base < TILE ? (int)(a.n - base) : TILE;
     }
@@ -541,19 +545,19 @@ __global__ __launch_bounds__(256) void k_sort_scatter(SortArgs a) {
         dig[r] = LO ? (uint32_t)lo[r] & 255u : (hi[r] >> a.shift) & 255u;
     }
     // where the tile's run of digit tid starts
-    uint32_t start;
+    uint32_t before = 0, tot = 0;
     if (SEG) {
-        start = a.hist[(int64_t)b * 256 + tid];
+        before = seg_start + a.hist[(int64_t)b * 256 + tid];
+        tot = a.dig_tot[seg * 256 + tid];
     } else {
-        uint32_t before = 0, tot = 0;
 #pragma unroll 16
         for (int t = 0; t < a.nblk; ++t) {
             const uint32_t v = a.hist[t * 256 + tid];
             before += t < b ? v : 0;
             tot += v;
         }
-        start = block256_excl_scan(tot, lds, nullptr) + before;
     }
+    const uint32_t start = block256_excl_scan(tot, lds, nullptr) + before;
     const uint32_t toff = tile_ranks<IPT>(dig, nmine, wcnt, lds, rk, 8);
     gbase[tid] = start - toff;
     __syncthreads();
@@ -733,7 +737,8 @@ __global__ __launch_bounds__(256) void k_gather_parts(const uint4* __restrict__ 
 template <int IPT, int LO, bool IDENT, bool KEYOUT, bool SEG>
 static void sort_pass(const SortArgs& a, unsigned nblk, bool counted, hipStream_t s) {
     if (!counted) k_sort_hist<IPT, LO, SEG><<<dim3(nblk), dim3(256), 0, s>>>(a);
-    if (SEG) k_sort_segscan<256 * IPT><<<dim3(kSegs), dim3(1024), 0, s>>>(a);
+    if (SEG && a.n < kScanWide) k_sort_segscan<256 * IPT, 128><<<dim3(kSegs, 2), dim3(1024), 0, s>>>(a);
+    else if (SEG) k_sort_segscan<256 * IPT, 32><<<dim3(kSegs, 8), dim3(1024), 0, s>>>(a);
     k_sort_scatter<IPT, LO, IDENT, KEYOUT, SEG><<<dim3(nblk), dim3(256), 0, s>>>(a);
 }
 
@@ -772,8 +777,9 @@ static void sort_segments(Ctx& c, const uint32_t* pos, const int8_t* species, ui
     uint32_t *ha = (uint32_t*)c.keys1, *hb = ha + c.cap_n;
     uint8_t* lo8 = (uint8_t*)c.keys0;
     uint32_t *v0 = (uint32_t*)c.vals0, *v1 = (uint32_t*)c.vals1;
-    uint32_t* tot = c.hist;  // kSegs totals, then the counts
-    uint32_t* hist = c.hist + kSegs;
+    uint32_t* tot = c.hist;  // kSegs totals, 256 of each segment, then the counts
+    uint32_t* dig = c.hist + kSegs;
+    uint32_t* hist = dig + kSegs * 256;
     k_part_hist<<<dim3(npart), dim3(256), 0, s>>>(pos, n, hist, npart);
     k_part_scan<<<dim3(kSegs), dim3(1024), 0, s>>>(hist, npart, tot);
     k_part_scatter<<<dim3(npart), dim3(256), 0, s>>>(pos, species, n, hist, npart, tot, rec, lo8, ha);
@@ -781,6 +787,7 @@ static void sort_segments(Ctx& c, const uint32_t* pos, const int8_t* species, ui
     a.n = n;
     a.hist = hist;
     a.seg_tot = tot;
+    a.dig_tot = dig;
     a.hi_in = ha; a.hi_out = hb; a.lo_in = lo8; a.val_out = v1;
     sort_pass<IPT, 8, true, true, true>(a, nblk, false, s);
     for (int p = 0; p < 3; ++p) {  // d1, d2, d3
@@ -795,7 +802,7 @@ static void sort_segments(Ctx& c, const uint32_t* pos, const int8_t* species, ui
 
 // Counts: the small path's kSmallTiles tiles, or the segments' tiles and totals (tiles of 2048 at least), or the
 // partition's tiles.
-int64_t sort_hist_size(int64_t cap) { return (cap / (256 * kSmallIpt) + kSegs + 1) * 256 + kSegs; }
+int64_t sort_hist_size(int64_t cap) { return (cap / (256 * kSmallIpt) + 2 * kSegs + 1) * 256 + kSegs; }
 
 hipError_t sort_particles(Ctx& c, const uint32_t* pos, const int8_t* species, int64_t n, int32_t* ts, int32_t* cells,
                           hipStream_t s) {
