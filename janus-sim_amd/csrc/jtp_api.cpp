@@ -562,26 +562,33 @@ static int check_status(Ctx& c, int64_t n) {
     return JTP_OK;
 }
 
-// What an evaluation needs beyond a mesh solve (contexts that only solve never pay for it): the particle buffers, the half
-// spectrum of the second mesh and the FP64 walk's polynomials.
-static int prepare(Ctx& c, int64_t n) {
-    if (c.p.interlace && c.p.pm_enabled && !c.spec2) {
-        const hipError_t e = dalloc_bytes(c.spec2, (size_t)c.G() * c.G() * c.Hc() * 2 * c.real_size());
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            return fail(&c, JTP_ERR_ALLOC, std::string("device allocation failed: ") + hipGetErrorString(e));
-        }
-    }
-    if (c.poly64.ok && !c.dev_fit64) {
-        JTP_HIP(&c, dalloc(c.dev_fit64, 1));
-        JTP_HIP(&c, hipMemcpy(c.dev_fit64, &c.poly64, sizeof(SplitPoly64), hipMemcpyHostToDevice));
-    }
+static int prepare_particles(Ctx& c, int64_t n) {
     const int64_t old_cap = c.cap_n;
     int rc = ensure_capacity(c, n);
     if (rc != JTP_OK) return rc;
     if (c.cap_n != old_cap) c.graph_dirty = true;  // buffers moved
     c.n_groups_max = (n + c.p.group_size - 1) / c.p.group_size + 4096;
     return JTP_OK;
+}
+
+// What an evaluation needs beyond a mesh solve or initial conditions (contexts that make no other call never pay for it): the
+// particle buffers, the half spectrum of the second mesh and the tables of the FP64 walk.
+static int prepare(Ctx& c, int64_t n) {
+    hipError_t e = hipSuccess;
+    if (c.p.interlace && c.p.pm_enabled && !c.spec2)
+        e = dalloc_bytes(c.spec2, (size_t)c.G() * c.G() * c.Hc() * 2 * c.real_size());
+    if (e == hipSuccess && c.p.tree_enabled && c.poly64.ok && !c.dev_fit64) {
+        SplitPoly64* d = nullptr;  // kept once it holds the tables
+        e = dalloc(d, 1);
+        if (e == hipSuccess) e = hipMemcpy(d, &c.poly64, sizeof(SplitPoly64), hipMemcpyHostToDevice);
+        if (e == hipSuccess) c.dev_fit64 = d;
+        else if (d) (void)hipFree(d);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(&c, JTP_ERR_ALLOC, std::string("device allocation failed: ") + hipGetErrorString(e));
+    }
+    return prepare_particles(c, n);
 }
 
 int jtp_compute_forces(jtp_ctx* h, int64_t n, const uint32_t* d_pos, const int8_t* d_species, void* d_acc,
@@ -759,7 +766,7 @@ int jtp_generate_ics(jtp_ctx* h, const jtp_ic_params* p, uint32_t* d_pos, void* 
         return fail(&c, JTP_ERR_ARG, "bad IC parameters");
     if (!d_pos || !d_vel || !d_species) return fail(&c, JTP_ERR_ARG, "null device pointer");
     const int64_t n = c.G3();
-    int rc = prepare(c, n);  // sort buffers for the sign keys
+    int rc = prepare_particles(c, n);  // sort buffers for the sign keys
     if (rc != JTP_OK) return rc;
     if (!c.grad) JTP_HIP(&c, dalloc_bytes(c.grad, (size_t)n * c.real_size()));  // third displacement grid
     const int64_t n_plus = (int64_t)std::llround((double)n / (1.0 + p->mu));  // ic_gen.rs:58-60
