@@ -2,7 +2,7 @@
 // the phase sequence of one force evaluation.
 //
 // Phase order on the caller's stream (each phase bracketed by a HIP event):
-//   keys + radix sort + particle gather | Karras tree + monopoles + groups |
+//   keys + radix sort + particle gather | radix tree + monopoles + groups |
 //   CIC deposit | FFT Poisson solve | interpolation | group walk (+ PM add, scatter to caller order)
 // The reference runs the same pieces with a device synchronisation after
 // every launch (src/nbody_gpu_twopass.rs:4486-4649); here only the final

@@ -39,8 +39,8 @@ constexpr int kCtrStatus = kCtrInter + 4;           // words that the host reads
 constexpr int kCtrXcd = 64;                         // kXcds walk-queue heads, kCtrXcdStride apart
 constexpr int kCtrXcdStride = 64;                   // 256 bytes: their atomics do not share a line
 constexpr int kCtrTotal = kCtrXcd + kXcds * kCtrXcdStride;
-// Walk groups whose smallest enclosing Morton cell holds more than kEarlySpan times the group's particles are walked
-// first (k_groups); groups[g].y carries the mark.
+// Walk groups whose smallest enclosing Morton cell reaches at least kEarlySpan / 2 group sizes of particles beyond them on one
+// side are walked first (k_groups); groups[g].y carries the mark.
 constexpr int kEarlySpan = 64;
 constexpr int32_t kEarlyMark = 1 << 30;
 inline int64_t early_cap(int64_t cap) { return cap / 256 + 4096; }  // entries of the list (beyond it: no mark)

@@ -100,7 +100,8 @@ __device__ inline void write_mono(int32_t p, const NodeSum& s, const uint32_t mn
 // is the right child of its parent if d(f - 1) > d(l) and the left child otherwise, and the parent's split lies at that
 // neighbour pair.  So a run that is complete needs two prefix lengths to know where it belongs, the two children of a
 // parent meet at the parent's split, and the node's number is known with its side: f for a right child, l for a left
-// one (0 for the root), as in Karras's construction.
+// one (0 for the root), as in Karras's construction.  (Agglomerative construction: Apetrei, Fast and Simple Agglomerative LBVH
+// Construction, 2014.)
 //
 // One workgroup holds up to kBtM consecutive items (leaves or finished subtrees) in LDS.  Every thread starts from its
 // item and climbs: it leaves its run at the parent's split; the second of the two to arrive merges and climbs on.
@@ -597,8 +598,8 @@ __global__ __launch_bounds__(1024) void k_group_offsets(int32_t n, int gs, int32
 // The groups, and the list of those to walk first.  A run of Morton-consecutive particles that straddles the boundary of a
 // large cell has a box that can reach across a dense region it has no part in; such a group opens everything there and
 // takes up to 16 ms beside a mean of 0.22 (2.2e7 clustered particles), and whatever was pulled last set the end of the
-// launch.  Their smallest enclosing Morton cell holds many times the group's particles (the keys kEarlySpan / 2 group
-// sizes before and after the run tell; in a level-4 cell with fewer particles than that none does), which also marks
+// launch.  Their smallest enclosing Morton cell reaches far beyond them (the keys kEarlySpan / 2 group sizes before and after
+// the run tell; in a level-4 cell with fewer particles than that none does), which also marks
 // ~3 % of harmless groups; with all of those first, the long ones overlap the rest.  Walk before -> after: 1.76 ->
 // 1.46 ms (1000003 clustered particles), 13.9 -> 12.7 (2.75e6, FP64), 39.0 -> 37.9 (2.2e7).
 __global__ void k_groups(const uint64_t* __restrict__ keys, int64_t n, const int32_t* __restrict__ cell4,
