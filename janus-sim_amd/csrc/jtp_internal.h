@@ -104,7 +104,7 @@ struct SplitPoly {
 //    it); beyond, x erfcx(x) as a polynomial of 1 / x^2;
 //  * exp(-x^2) = 2^n (1 + f Q(f)), n + f = -x^2 / ln 2, |f| <= 1/2 (Cody and Waite's reduction, with the product kept exact by
 //    an FMA).
-// Error relative to the pair's own force, against 128-bit arithmetic: at most 7e-16 at every x, rms 1.6e-16 (erfc and exp of
+// Error relative to the pair's own force, against 128-bit arithmetic: at most 7e-16 at every x, rms 1.9e-16 (erfc and exp of
 // a rounded x: 3.0e-15 for x <= 2.25, 8.3e-15 for x <= 4, 2.4e-14 for x <= 6.2; rms 4e-16, 1.4e-15, 5.7e-15).  1 / rho^3 plus a
 // polynomial, at 44 instructions a cut pair instead of 71, loses digits as S falls: 2.7e-14 at 2.25, 3e-9 at 4.
 // `ok`: the pairs' range covers r_cut (up to 5.4 r_s) and the polynomials, evaluated in double, are within kFit64Tol of
