@@ -135,7 +135,7 @@ struct Pair<float, MODE, CUT> {
 };
 
 // 1 / v^{3/2}, v > 0, within half an ulp and 2^-58: the hardware's estimate of 1 / sqrt(v) (within 2^-20) cut to 17 bits, y,
-// so that y^2 and y^3 are exact, times the series of (1 - e)^{-3/2} in the residual e = 1 - v y^2 < 2^-14.
+// so that y^2 and y^3 are exact, times the series of (1 - e)^{-3/2} in the residual e = 1 - v y^2 < 1.07 x 2^-15.
 __device__ inline double inv_cube(double v) {
     const double y = __hiloint2double(__double2hiint(__builtin_amdgcn_rsq(v)) & ~15, 0);
     const double w = y * y, e = __builtin_fma(-v, w, 1.0), y3 = w * y;
